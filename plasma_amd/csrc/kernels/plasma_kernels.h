@@ -57,6 +57,11 @@ int plasma_kern_tile2lapack(plasma_enum_t region, plasma_desc_t A, void *pA,
  */
 int plasma_kern_potrf_diag(plasma_enum_t uplo, plasma_desc_t A, int k,
                            void *inv, int *status, hipStream_t s);
+/* The same for real tiles of order mb <= 128 (plasma_diag128_ok), the whole
+ * tile in LDS; plasma_kern_potrf_diag calls it where it applies. */
+int plasma_diag128_ok(plasma_desc_t A);
+int plasma_kern_diag128(plasma_enum_t uplo, plasma_desc_t A, int k, void *inv,
+                        int *status, hipStream_t s);
 
 /* Diagonal tile k factored with only the inverses of its 32 x 32 diagonal
  * blocks written to W_kk (the rest of W_kk is left as it was), for the

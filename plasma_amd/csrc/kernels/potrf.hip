@@ -1087,6 +1087,8 @@ extern "C" int plasma_kern_potrf_diag(plasma_enum_t uplo, plasma_desc_t A,
                                       int k, void *inv, int *status,
                                       hipStream_t s)
 {
+    if (plasma_diag128_ok(A))
+        return plasma_kern_diag128(uplo, A, k, inv, status, s);
     if (A.precision == PlasmaRealDouble)
         return launch_potrf_diag<double>(uplo, A, k, 1, 1, inv, status, s);
     if (A.precision == PlasmaRealFloat)
