@@ -226,7 +226,8 @@ static int k_update(const group_t *g, int pbase, int ncols, int n0, int n1,
         err = plasma_kern_trailing_update_split(
             g->uplo, g->A, pbase, kdepth, n0, n1, panel, planes_of(g, panel),
             g->pcols, copy_cols, max_wgs, g->split == SPLIT_BF16X1, g->st, s);
-    else if (update64_on() && plasma_update64_ok(g->A, kdepth))
+    else if (update64_on() && plasma_update64_ok(g->A, kdepth) &&
+             !plasma_direct_update_ok(g->A, n0, n1))
         err = plasma_kern_trailing_update64(g->uplo, g->A, pbase, kdepth, n0,
                                             n1, panel, g->pcols, copy_cols,
                                             max_wgs, g->st, s);

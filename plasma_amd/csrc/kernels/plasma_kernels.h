@@ -130,6 +130,10 @@ int plasma_kern_trailing_update(plasma_enum_t uplo, plasma_desc_t A,
                                 int copy_cols, int max_wgs,
                                 const int *status, hipStream_t s);
 
+/* Whether the update of columns [n_first, n_end) has so few blocks that
+ * plasma_kern_trailing_update runs it in small ones (directgemm.hip.h). */
+int plasma_direct_update_ok(plasma_desc_t A, int n_first, int n_end);
+
 /*
  * Triangular sweeps of potrs (reference pztrsm.c:113-177 and :43-107).
  * backward == 0: solve L Y = B (forward); backward == 1: L^T X = Y.

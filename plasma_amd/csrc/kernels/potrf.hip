@@ -9,6 +9,7 @@
 // common.hip.h (upper storage is read as L = U^T).
 #include "common.hip.h"
 #include "tilegemm.hip.h"
+#include "directgemm.hip.h"
 #include "plasma_kernels.h"
 
 namespace {
@@ -555,7 +556,7 @@ __global__ __launch_bounds__(NT, MINB) void potrf_diag_kernel(
 // ---------------------------------------------------------------------------
 
 // Trailing update by the panels of a column group: tiles (m, n) of columns
-// [n_first, ...) enumerated column by column, bpt x bpt blocks of 128 per
+// [n_first, ...) enumerated column by column, bpt x bpt blocks of BM rows per
 // tile, C(m, n) -= P(m) P(n)^T with P(m) the first `kdepth` columns of the
 // group's panel buffer tile m (at panel + (m - pbase - 1) * mb * pcols,
 // column major, ld = mb; its columns [j * nb, (j + 1) * nb) hold the solved
@@ -563,7 +564,7 @@ __global__ __launch_bounds__(NT, MINB) void potrf_diag_kernel(
 // either storage triangle.  The first `ncopy` workgroups copy panel columns
 // back into A(m, pbase + j), m > pbase + j, j < ncols, instead (transposed
 // for upper storage).
-template <typename T>
+template <typename T, int BM = tg::BM>
 struct UpdateDecode {
     plasma_desc_t A;
     int pbase, pcols, kdepth, ncols, n_first, bpt, upper, ncopy;
@@ -612,7 +613,7 @@ struct UpdateDecode {
         trapezoid_decode(b / per_tile, A.mt, n_first, &m, &n);
         if (m == n && bj > bi) return false;
         const int mv = plasma_tile_mview(A, m), nv = plasma_tile_mview(A, n);
-        const int r0 = bi * tg::BM, c0 = bj * tg::BM;
+        const int r0 = bi * BM, c0 = bj * BM;
         if (r0 >= mv || c0 >= nv) return false;
         j.X = sub(panel_tile(m), r0, 0);
         j.Y = sub(panel_tile(n), c0, 0);
@@ -629,7 +630,7 @@ struct UpdateDecode {
 // Panel solve of step k: P(m) = A(m,k) W_kk^T for m > k into column block
 // `pcol` of the panel buffer tile m (at panel + (m - pbase - 1) * mb * pcols
 // + pcol * mb, column major, ld = mb).
-template <typename T>
+template <typename T, int BM = tg::BM>
 struct PanelDecode {
     plasma_desc_t A;
     int k, bpt, upper, pbase, pcols, pcol;
@@ -642,7 +643,7 @@ struct PanelDecode {
         const int sub_ = b % per_tile;
         const int bi = sub_ / bpt, bj = sub_ % bpt;
         const int mv = plasma_tile_mview(A, m), nb = plasma_tile_mview(A, k);
-        const int r0 = bi * tg::BM, c0 = bj * tg::BM;
+        const int r0 = bi * BM, c0 = bj * BM;
         if (r0 >= mv || c0 >= nb) return false;
         View<T> W;
         W.p = const_cast<T *>(inv) + (size_t)k * A.mb * A.mb;
@@ -658,7 +659,7 @@ struct PanelDecode {
         j.C = sub(S, r0, c0);
         j.xrows = mv - r0;
         j.yrows = nb - c0;
-        j.K = nb;
+        j.K = min(nb, c0 + BM);         // W_kk is lower triangular
         j.lower = false;
         j.diag_off = 0;
         return true;
@@ -829,6 +830,47 @@ int launch_panel_blocked(plasma_enum_t uplo, plasma_desc_t A, int k,
     return hipGetLastError() == hipSuccess ? 0 : PlasmaErrorInternal;
 }
 
+// Block width of the direct kernel (directgemm.hip.h) for a launch of n128
+// 128 x 128 blocks, in units of 32; 0: the staged kernels.  Up to DG_32 of
+// them even 64 x 64 blocks leave most CUs idle; beyond DG_64 (two rounds of
+// the chip's workgroup slots) the staged kernels' smaller operand traffic
+// counts.  FP64 solves (nrhs 64 / 10 / 1): n = 500 512 us with the staged
+// kernels alone, 444 with 64 x 64 blocks, 437 with both widths; n = 2049
+// 2186, 1762, 1734 us; n = 8192 12.6, 10.1, 10.0 ms.  DG_64 = 512: n = 16384
+// 40.3 ms, 1024: 40.1, 2048: 40.0 (staged alone 44.0); DG_32 = 64: n = 8192
+// 10.2 ms.  One launch at n = 8192: panel 28.6 -> 16.8 us beside the bulk
+// update, next column's update (K = 128) 27 -> 12 us.
+constexpr long DG_32 = 24, DG_64 = 1024;
+
+int dg_width(long n128)
+{
+    return n128 <= DG_32 ? 1 : n128 <= DG_64 ? 2 : 0;
+}
+
+// The direct kernel over the jobs of a decoder with blocks of 32 FW, `tiles`
+// tiles of mb x mb and ncopy copy jobs.  make(blocks per tile side) builds
+// the decoder.  CL: C has unit row stride also for upper storage (the panel
+// buffer).
+template <typename T, int FW, template <typename, int> class Dec, bool ACC,
+          bool CL, typename Make>
+void launch_direct(bool up, long tiles, int mb, const int *status,
+                   hipStream_t s, Make make, int ncopy = 0)
+{
+    typedef Dec<T, 32 * FW> D;
+    const int bpt = (mb + 32 * FW - 1) / (32 * FW);
+    const int njobs = (int)(tiles * bpt * bpt) + ncopy;
+    const D d = make(bpt);
+    const dim3 grid(tg::xcd_grid(njobs)), block(dg::NT);
+    // the panel solve reads A itself (contiguous k in upper storage), the
+    // update both operands from the panel buffer
+    if (up)
+        hipLaunchKernelGGL((dg::kernel<T, FW, CL, ACC, ACC, true, D>), grid,
+                           block, 0, s, d, njobs, status);
+    else
+        hipLaunchKernelGGL((dg::kernel<T, FW, true, ACC, true, true, D>),
+                           grid, block, 0, s, d, njobs, status);
+}
+
 template <typename T>
 int launch_trsm_panel(plasma_enum_t uplo, plasma_desc_t A, int k,
                       const void *inv, void *panel, int pbase, int pcols,
@@ -836,19 +878,36 @@ int launch_trsm_panel(plasma_enum_t uplo, plasma_desc_t A, int k,
 {
     const int ntiles = A.mt - k - 1;
     if (ntiles <= 0) return 0;
+    const bool up = uplo == PlasmaUpper;
     const int bpt = (A.mb + tg::BM - 1) / tg::BM;
-    PanelDecode<T> d{A, k, bpt, uplo == PlasmaUpper, pbase, pcols, pcol,
-                     (const T *)inv, (T *)panel};
-    if (uplo == PlasmaUpper)
+    const int n128 = ntiles * bpt * bpt;
+    if (dg_width(n128)) {
+        if (dg_width(n128) == 1)
+            launch_direct<T, 1, PanelDecode, false, true>(
+                up, ntiles, A.mb, status, s, [&](int bp) {
+                    return PanelDecode<T, 32>{A, k, bp, up, pbase, pcols, pcol,
+                                              (const T *)inv, (T *)panel};
+                });
+        else
+            launch_direct<T, 2, PanelDecode, false, true>(
+                up, ntiles, A.mb, status, s, [&](int bp) {
+                    return PanelDecode<T, 64>{A, k, bp, up, pbase, pcols, pcol,
+                                              (const T *)inv, (T *)panel};
+                });
+        return hipGetLastError() == hipSuccess ? 0 : PlasmaErrorInternal;
+    }
+    PanelDecode<T> d{A, k, bpt, up, pbase, pcols, pcol, (const T *)inv,
+                     (T *)panel};
+    if (up)
         hipLaunchKernelGGL((tg::kernel<T, true, false, false, false, true,
                                        PanelDecode<T>>),
-                           dim3(tg::xcd_grid(ntiles * bpt * bpt)),
-                           dim3(tg::NT), 0, s, d, ntiles * bpt * bpt, status);
+                           dim3(tg::xcd_grid(n128)), dim3(tg::NT), 0, s, d,
+                           n128, status);
     else
         hipLaunchKernelGGL((tg::kernel<T, true, false, false, true, true,
                                        PanelDecode<T>>),
-                           dim3(tg::xcd_grid(ntiles * bpt * bpt)),
-                           dim3(tg::NT), 0, s, d, ntiles * bpt * bpt, status);
+                           dim3(tg::xcd_grid(n128)), dim3(tg::NT), 0, s, d,
+                           n128, status);
     return hipGetLastError() == hipSuccess ? 0 : PlasmaErrorInternal;
 }
 
@@ -870,6 +929,25 @@ int launch_trailing_update(plasma_enum_t uplo, plasma_desc_t A, int pbase,
     int ncopy = 0;
     for (int j = 0; j < copy_cols; j++)
         ncopy += max(A.mt - (pbase + j) - 1, 0);
+    const long tiles = nblocks / (bpt * bpt);
+    if (dg_width(nblocks) && nblocks > 0) {
+        const bool up = uplo == PlasmaUpper;
+        if (dg_width(nblocks) == 1)
+            launch_direct<T, 1, UpdateDecode, true, false>(
+                up, tiles, A.mb, status, s, [&](int bp) {
+                    return UpdateDecode<T, 32>{A, pbase, pcols, kdepth,
+                                               max(copy_cols, 1), n_first, bp,
+                                               up, ncopy, (const T *)panel};
+                }, ncopy);
+        else
+            launch_direct<T, 2, UpdateDecode, true, false>(
+                up, tiles, A.mb, status, s, [&](int bp) {
+                    return UpdateDecode<T, 64>{A, pbase, pcols, kdepth,
+                                               max(copy_cols, 1), n_first, bp,
+                                               up, ncopy, (const T *)panel};
+                }, ncopy);
+        return hipGetLastError() == hipSuccess ? 0 : PlasmaErrorInternal;
+    }
     nblocks += ncopy;
     if (nblocks == 0) return 0;
     if (nblocks > 0x7fffffffL) return PlasmaErrorNotSupported;
@@ -1159,6 +1237,15 @@ extern "C" int plasma_kern_trsm_panel(plasma_enum_t uplo, plasma_desc_t A,
         return launch_trsm_panel<float>(uplo, A, k, inv, panel, pbase, pcols,
                                         pcol, status, s);
     return PlasmaErrorNotSupported;
+}
+
+extern "C" int plasma_direct_update_ok(plasma_desc_t A, int n_first, int n_end)
+{
+    n_end = min(n_end, A.mt);
+    long ntiles = 0;
+    for (int n = n_first; n < n_end; n++) ntiles += A.mt - n;
+    const long bpt = (A.mb + tg::BM - 1) / tg::BM;
+    return ntiles > 0 && dg_width(ntiles * bpt * bpt) != 0;
 }
 
 extern "C" int plasma_kern_trailing_update(plasma_enum_t uplo,
