@@ -433,7 +433,7 @@ int plasma_dhposv(plasma_enum_t uplo, int n, int nrhs, double *pA, int lda,
         fallback = 1;
     }
     else {
-        d.mpan = plasma_rsolve_prepare(uplo, As, d.inv_s, &sequence,
+        d.mpan = plasma_rsolve_prepare(uplo, As, nrhs, d.inv_s, &sequence,
                                        &request);
         /* X = M^{-1} S B, then refinement steps */
         precond(&d, B, X, &sequence, &request);

@@ -212,7 +212,7 @@ static void omp_mixed(plasma_enum_t hi, plasma_enum_t lo, plasma_enum_t uplo,
     plasma_pxpotrf(uplo, As, inv_s, sequence, request);
     /* the refinement solves with this factor up to 31 times: prepare its
      * repeated-solve form once (super-block inverses or scaled panels) */
-    mpan = plasma_rsolve_prepare(uplo, As, inv_s, sequence, request);
+    mpan = plasma_rsolve_prepare(uplo, As, nrhs, inv_s, sequence, request);
     solve_s(uplo, As, Xs, inv_s, mpan, sequence, request);
     if (lag2_step(Xs, X, st, s, sequence, request))
         goto done;

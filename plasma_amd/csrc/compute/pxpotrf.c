@@ -680,6 +680,34 @@ void plasma_pxtrsm_left(plasma_enum_t uplo, plasma_enum_t trans,
     plasma_dev_free(scratch);
 }
 
+/* Both sweeps of potrs, each in one launch (kernels/flowsweep.hip).
+ * Returns 0 when the path does not apply (the per-step sweeps run). */
+static int flow_sweeps(plasma_enum_t uplo, plasma_desc_t A, plasma_desc_t B,
+                       const void *inv, plasma_sequence_t *sequence,
+                       plasma_request_t *request)
+{
+    if (B.mb != A.mb || !plasma_flow_sweep_ok(A, B.n))
+        return 0;
+    plasma_context_t *ctx = plasma_context_self();
+    hipStream_t s0 = ctx->stream;
+    const size_t n = plasma_flow_sweep_ints(B);
+    int *sync = plasma_dev_alloc(2 * n * sizeof(int));
+    if (sync == NULL)
+        return 0;
+    int *st = plasma_sequence_dstatus(sequence, request);
+    int slot;
+    plasma_prof_begin(s0, PlasmaProfSweep, 2.0 * B.m * B.m * B.n, 0, &slot);
+    if (!issue(plasma_kern_fill_int(sync, 0, (int)(2 * n), s0), sequence,
+               request) &&
+        !issue(plasma_kern_flow_sweep(uplo, 0, A, B, inv, sync, st, s0),
+               sequence, request))
+        issue(plasma_kern_flow_sweep(uplo, 1, A, B, inv, sync + n, st, s0),
+              sequence, request);
+    plasma_prof_end(s0, slot);
+    plasma_dev_free(sync);
+    return 1;
+}
+
 void plasma_pxpotrs(plasma_enum_t uplo, plasma_desc_t A, plasma_desc_t B,
                     const void *inv, plasma_sequence_t *sequence,
                     plasma_request_t *request)
@@ -707,6 +735,10 @@ void plasma_pxpotrs(plasma_enum_t uplo, plasma_desc_t A, plasma_desc_t B,
         inv = own_inv;
     }
     /* reference compute/zpotrs.c:270-283 */
+    if (flow_sweeps(uplo, A, B, inv, sequence, request)) {
+        plasma_dev_free(own_inv);
+        return;
+    }
     plasma_pxtrsm_left(uplo, uplo == PlasmaUpper ? PlasmaConjTrans
                                                  : PlasmaNoTrans,
                        A, B, inv, sequence, request);
@@ -883,15 +915,23 @@ void plasma_pxpotrs_sb(plasma_enum_t uplo, plasma_desc_t A, plasma_desc_t B,
     plasma_dev_free(Y);
 }
 
-/* The repeated-solve form of a factor: the super-block inverses when those
- * sweeps apply, else the scaled panels; NULL when the block could not be
- * allocated (plasma_rsolve then runs the plain sweeps). */
-void *plasma_rsolve_prepare(plasma_enum_t uplo, plasma_desc_t A,
+/* The repeated-solve form of a factor for nrhs right-hand sides: the
+ * super-block inverses when those sweeps apply, else the scaled panels; NULL
+ * when none is needed or the block could not be allocated (plasma_rsolve then
+ * runs the sweeps of plasma_pxpotrs). */
+void *plasma_rsolve_prepare(plasma_enum_t uplo, plasma_desc_t A, int nrhs,
                             const void *inv, plasma_sequence_t *sequence,
                             plasma_request_t *request)
 {
     /* complex factors are solved by the plain sweeps */
     if (plasma_is_complex(A.precision))
+        return NULL;
+    /* up to 16 right-hand sides the dataflow sweeps read L once per sweep
+     * and need no preparation: dsposv n = 4000, nrhs 8: 3692 -> 3267 us, n =
+     * 7932, nrhs 4: 9.25 -> 7.96 ms, n = 32768, nrhs 16: 89.7 -> 83.7 ms.
+     * Every further 16 read it again: nrhs 64, n = 4096 3907 -> 4005 us, n =
+     * 8192 8.53 -> 8.94 ms, n = 32768 83.2 -> 91.9 ms */
+    if (nrhs <= FLOW_SWEEP_RSOLVE && plasma_flow_sweep_ok(A, nrhs))
         return NULL;
     const int sb = plasma_sweep_tiles(A) > 0;
     void *form = plasma_dev_alloc(sb ? plasma_sbinv_bytes(A)

@@ -248,7 +248,7 @@ void plasma_pxpbtrs(plasma_enum_t uplo, plasma_desc_t A, plasma_desc_t B,
                     plasma_request_t *request);
 /* Either form for a factor solved many times: rsolve_prepare computes it
  * into one pool block (NULL: none, the plain sweeps run), rsolve solves. */
-void *plasma_rsolve_prepare(plasma_enum_t uplo, plasma_desc_t A,
+void *plasma_rsolve_prepare(plasma_enum_t uplo, plasma_desc_t A, int nrhs,
                             const void *inv, plasma_sequence_t *sequence,
                             plasma_request_t *request);
 void plasma_rsolve(plasma_enum_t uplo, plasma_desc_t A, plasma_desc_t B,

@@ -101,7 +101,7 @@ template <typename T, int FW, bool UNIT> struct Operand {
                 for (int i = 0; i < FW; i++) g.v[i][v] = at<T>(qv, off[i]);
             }
         }
-        else if (vec) {
+        else if (vec && kc % V == 0) {
 #pragma unroll
             for (int i = 0; i < FW; i++) {
                 const vec_t x = at<vec_t>(q, off[i]);

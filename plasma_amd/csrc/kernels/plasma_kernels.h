@@ -135,6 +135,21 @@ int plasma_kern_trailing_update(plasma_enum_t uplo, plasma_desc_t A,
 int plasma_direct_update_ok(plasma_desc_t A, int n_first, int n_end);
 
 /*
+ * One sweep of potrs in one launch (real tiles of order <= 128 and at most
+ * FLOW_SWEEP_NRHS right-hand sides: plasma_flow_sweep_ok): L Y = B forward,
+ * L^T X = Y backward, B overwritten.  sync: plasma_flow_sweep_ints(B) ints,
+ * zero before the launch.  Up to FLOW_SWEEP_RSOLVE right-hand sides it is
+ * also the form for a factor that is solved with many times.
+ */
+#define FLOW_SWEEP_NRHS 128
+#define FLOW_SWEEP_RSOLVE 16
+int plasma_flow_sweep_ok(plasma_desc_t A, int nrhs);
+size_t plasma_flow_sweep_ints(plasma_desc_t B);
+int plasma_kern_flow_sweep(plasma_enum_t uplo, int backward, plasma_desc_t A,
+                           plasma_desc_t B, const void *inv, int *sync,
+                           const int *status, hipStream_t s);
+
+/*
  * Triangular sweeps of potrs (reference pztrsm.c:113-177 and :43-107).
  * backward == 0: solve L Y = B (forward); backward == 1: L^T X = Y.
  * trsm_diag_left computes S = W_kk B(k,:) (forward) or W_kk^T B(k,:)
