@@ -115,6 +115,59 @@ static int vbatched_grid(plasma_context_t *ctx, plasma_enum_t precision,
     return grid > batch ? batch : grid;
 }
 
+/* Class of a system's order: 0 above 256, 1 above 128, 2 */
+static int order_class(int n)
+{
+    return n > 256 ? 0 : n > 128 ? 1 : 2;
+}
+
+/* The class launches of up to 16 right-hand sides: the largest class on the
+ * main stream, the others beside it on the panel stream (their workgroups
+ * fill the CUs its last systems leave idle), joined on return. */
+static int vbatched16(plasma_context_t *ctx, plasma_enum_t precision,
+                      int upper, int batch, const int count[3], const int *n,
+                      void *A, const size_t *aoff, void *W, int nrhs, void *B,
+                      const size_t *boff, int *info, const int *order,
+                      int *ticket)
+{
+    const int cls[2] = {count[0], count[0] + count[1]};
+    void *w[3];
+    char *p = W;
+    for (int k = 0; k < 3; k++) {
+        w[k] = p;
+        if (p != NULL && count[k] > 0)
+            p += plasma_vbatched16_bytes(precision, k, count[k],
+                                         ctx->num_cus);
+    }
+    const int fork = (count[0] > 0) && (count[1] + count[2] > 0);
+    hipStream_t s0 = ctx->stream, s1 = fork ? ctx->panel_stream : s0;
+    hipStream_t const s[3] = {s0, s1, s1};
+    hipEvent_t ev[2] = {NULL, NULL};
+    int err = 0;
+    if (fork) {
+        for (int k = 0; k < 2 && !err; k++)
+            err = plasma_hip_check(hipEventCreateWithFlags(
+                                       &ev[k], hipEventDisableTiming),
+                                   "hipEventCreate");
+        if (!err) {
+            hipEventRecord(ev[0], s0);
+            hipStreamWaitEvent(s1, ev[0], 0);
+        }
+    }
+    if (!err)
+        err = plasma_kern_vbatched16(precision, upper, batch, cls, n, A, aoff,
+                                     w, nrhs, B, boff, info, order, ticket,
+                                     ctx->num_cus, s);
+    if (fork && ev[1] != NULL) {
+        hipEventRecord(ev[1], s1);
+        hipStreamWaitEvent(s0, ev[1], 0);
+    }
+    for (int k = 0; k < 2; k++)
+        if (ev[k] != NULL)
+            hipEventDestroy(ev[k]);
+    return err ? PlasmaErrorInternal : 0;
+}
+
 static int vbatched(plasma_enum_t precision, plasma_enum_t uplo, int batch,
                     const int *n, void *A, const size_t *aoff, int nrhs,
                     void *B, const size_t *boff, int *info)
@@ -155,12 +208,14 @@ static int vbatched(plasma_enum_t precision, plasma_enum_t uplo, int batch,
         retval = PlasmaErrorInternal;
         goto done;
     }
+    int count[3] = {0, 0, 0};
     for (int i = 0; i < batch; i++) {
         if (hn[i] < 0 || hn[i] > VBATCH_NMAX) {
             plasma_error("illegal order of a system");
             retval = -3;
             goto done;
         }
+        count[order_class(hn[i])]++;
         ord[i].n = hn[i];
         ord[i].i = i;
     }
@@ -170,9 +225,17 @@ static int vbatched(plasma_enum_t precision, plasma_enum_t uplo, int batch,
 
     /* one resident grid, each workgroup with its own slab of W */
     const int grid = vbatched_grid(ctx, precision, batch);
-    W = plasma_dev_alloc((size_t)grid * plasma_kern_vbatched_wslab(precision));
+    const int classes = plasma_vbatched16_ok(nrhs);
+    size_t wbytes = (size_t)grid * plasma_kern_vbatched_wslab(precision);
+    if (classes) {
+        wbytes = 0;
+        for (int k = 0; k < 3; k++)
+            wbytes += plasma_vbatched16_bytes(precision, k, count[k],
+                                              ctx->num_cus);
+    }
+    W = plasma_dev_alloc(wbytes);
     dord = plasma_dev_alloc(nbytes);
-    dticket = plasma_dev_alloc(sizeof(int));
+    dticket = plasma_dev_alloc(3 * sizeof(int));
     if (W == NULL || dord == NULL || dticket == NULL) {
         retval = PlasmaErrorOutOfMemory;
         goto done;
@@ -198,13 +261,16 @@ static int vbatched(plasma_enum_t precision, plasma_enum_t uplo, int batch,
     if (plasma_hip_check(hipMemcpyAsync(dord, hord, nbytes,
                                         hipMemcpyHostToDevice, s),
                          "hipMemcpy(order)") ||
-        plasma_kern_fill_int(dticket, 0, 1, s) != 0) {
+        plasma_kern_fill_int(dticket, 0, 3, s) != 0) {
         retval = PlasmaErrorInternal;
         goto done;
     }
-    if (plasma_kern_vbatched_posv(precision, uplo == PlasmaUpper, batch, dn,
-                                  A, doff, W, nrhs, B, dboff, dinfo, dord,
-                                  dticket, grid, s) != 0) {
+    if (classes
+            ? vbatched16(ctx, precision, uplo == PlasmaUpper, batch, count, dn,
+                         A, doff, W, nrhs, B, dboff, dinfo, dord, dticket)
+            : plasma_kern_vbatched_posv(precision, uplo == PlasmaUpper, batch,
+                                        dn, A, doff, W, nrhs, B, dboff, dinfo,
+                                        dord, dticket, grid, s)) {
         retval = PlasmaErrorInternal;
         goto done;
     }
@@ -221,6 +287,7 @@ static int vbatched(plasma_enum_t precision, plasma_enum_t uplo, int batch,
 done:
     /* the host arrays below are freed only after the copies that read them
      * (also on the error paths) */
+    hipStreamSynchronize(ctx->panel_stream);
     hipStreamSynchronize(ctx->stream);
     if (own_n) plasma_dev_free(dn);
     if (own_off) plasma_dev_free(doff);
@@ -301,6 +368,7 @@ int plasma_dposv_vbatched_noalloc(plasma_enum_t uplo, int batch,
     const size_t obytes = (size_t)batch * sizeof(size_t);
     const int host_n = !plasma_is_device_ptr(n);
     const int *dn = n;
+    int count[3] = {0, 0, 0};
     if (host_n) {
         /* checked here, like plasma_dposv_vbatched, before any launch */
         for (int i = 0; i < batch; i++)
@@ -308,6 +376,8 @@ int plasma_dposv_vbatched_noalloc(plasma_enum_t uplo, int batch,
                 plasma_error("illegal order of a system");
                 return -3;
             }
+        for (int i = 0; i < batch; i++)
+            count[order_class(n[i])]++;
         if (plasma_hip_check(hipMemcpyAsync(r.n, n, nbytes,
                                             hipMemcpyHostToDevice, s),
                              "hipMemcpyAsync(n)"))
@@ -335,7 +405,7 @@ int plasma_dposv_vbatched_noalloc(plasma_enum_t uplo, int batch,
         return PlasmaErrorInternal;
     if (!host_n) {
         /* orders in device memory: checked by the order kernel */
-        int ctrl[2] = {0, 0};
+        int ctrl[4] = {0, 0, 0, 0};
         if (plasma_hip_check(hipMemcpyAsync(ctrl, r.ctrl, sizeof(ctrl),
                                             hipMemcpyDeviceToHost, s),
                              "hipMemcpyAsync(flag)") ||
@@ -345,6 +415,31 @@ int plasma_dposv_vbatched_noalloc(plasma_enum_t uplo, int batch,
             plasma_error("illegal order of a system");
             return -3;
         }
+        count[0] = ctrl[2];
+        count[1] = ctrl[3] - ctrl[2];
+        count[2] = batch - ctrl[3];
+    }
+    /* the class launches, when the slab area holds their workspace (they
+     * run one after the other and share it); a workgroup's results do not
+     * depend on the launch that holds it */
+    size_t wmax = 0;
+    for (int k = 0; k < 3; k++) {
+        const size_t w = plasma_vbatched16_bytes(PlasmaRealDouble, k, count[k],
+                                                 ctx->num_cus);
+        if (w > wmax)
+            wmax = w;
+    }
+    if (plasma_vbatched16_ok(nrhs) &&
+        wmax <= r.wslab_bytes * (size_t)r.grid_max) {
+        const int cls[2] = {count[0], count[0] + count[1]};
+        void *const w[3] = {r.W, r.W, r.W};
+        hipStream_t const ss[3] = {s, s, s};
+        if (plasma_kern_vbatched16(PlasmaRealDouble, uplo == PlasmaUpper,
+                                   batch, cls, dn, A, daoff, w, nrhs, B,
+                                   dboff, dinfo, r.order, r.ctrl + 4,
+                                   ctx->num_cus, ss) != 0)
+            return PlasmaErrorInternal;
+        goto copy_info;
     }
     int grid = vbatched_grid(ctx, PlasmaRealDouble, batch);
     if (grid > r.grid_max)
@@ -353,6 +448,7 @@ int plasma_dposv_vbatched_noalloc(plasma_enum_t uplo, int batch,
                                   batch, dn, A, daoff, r.W, nrhs, B, dboff,
                                   dinfo, r.order, r.ctrl, grid, s) != 0)
         return PlasmaErrorInternal;
+copy_info:
     if (host_info &&
         plasma_hip_check(hipMemcpyAsync(info, r.info, nbytes,
                                         hipMemcpyDeviceToHost, s),

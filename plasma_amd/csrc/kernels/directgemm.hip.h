@@ -52,8 +52,11 @@ template <typename T> __device__ __forceinline__ DG_GLOBAL T *uni(T *p)
 // (base + lane offset) of a loop into a 64-bit vector pointer of its own.
 template <typename P> __device__ __forceinline__ P scalar(P p)
 {
-    asm("" : "+s"(p));
-    return p;
+    const uint64_t v = (uint64_t)p;
+    uint64_t u = (uint64_t)(unsigned)uni((int)(v >> 32)) << 32 |
+                 (unsigned)uni((int)v);
+    asm("" : "+s"(u));
+    return (P)u;
 }
 
 // FW operand rows of a lane for one chunk

@@ -13,7 +13,8 @@
 //
 // Layout (byte offsets, each region 256-byte aligned):
 //   W      grid slabs of the diagonal-block inverses (FP64)
-//   ctrl   ticket, invalid-order flag
+//   ctrl   ticket, invalid-order flag, counts of the two larger classes of
+//          orders, a ticket per class
 //   n      orders (when the caller's array is on the host)
 //   order  the systems, largest order first
 //   info   per-system info (when the caller's array is on the host)
@@ -79,6 +80,12 @@ __global__ __launch_bounds__(ORDER_NT) void order_kernel(const int *n,
             start[v] = s;
             s += c;
         }
+    }
+    __syncthreads();
+    if (t == 0) {
+        ctrl[2] = start[256];      // systems of order > 256
+        ctrl[3] = start[128];      // > 128
+        for (int k = 4; k < 7; k++) ctrl[k] = 0;    // tickets of the classes
     }
     __syncthreads();
     for (int i = t; i < batch; i += ORDER_NT) {

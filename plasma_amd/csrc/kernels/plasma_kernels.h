@@ -209,6 +209,23 @@ int plasma_kern_vbatched_posv(plasma_enum_t precision, int upper, int batch,
                               void *W, int nrhs, void *B, const size_t *boff,
                               int *info, const int *order, int *ticket,
                               int grid, hipStream_t s);
+/*
+ * The same for at most 16 right-hand sides (plasma_vbatched16_ok), one launch
+ * per class of orders: systems [0, cls[0]) of `order` have n > 256, [cls[0],
+ * cls[1]) n > 128, the rest n <= 128.  ticket: one per class, zero on entry.
+ * Class k runs on s[k] with workspace W[k], plasma_vbatched16_bytes bytes for
+ * `count` systems on a device of `cus` CUs (the classes may share one block
+ * when they share a stream); unused without right-hand sides.
+ */
+int plasma_vbatched16_ok(int nrhs);
+size_t plasma_vbatched16_bytes(plasma_enum_t precision, int cls, int count,
+                               int cus);
+int plasma_kern_vbatched16(plasma_enum_t precision, int upper, int batch,
+                           const int cls[2], const int *n, void *A,
+                           const size_t *aoff, void *const W[3], int nrhs,
+                           void *B, const size_t *boff, int *info,
+                           const int *order, int *ticket, int cus,
+                           hipStream_t const s[3]);
 
 /*
  * Super-block sweeps (kernels/ssweep.hip), nb a multiple of 64, S tiles per
