@@ -18,42 +18,6 @@
 
 #define VBATCH_NMAX 512
 
-typedef struct {
-    int n, i;
-} order_t;
-
-static int by_n_desc(const void *a, const void *b)
-{
-    const order_t *x = a, *y = b;
-    if (x->n != y->n)
-        return y->n - x->n;
-    return x->i - y->i;
-}
-
-/* Device copy of a host or device array (owned copy in *dev_out).  The
- * copy goes on the context stream: pool memory is handed out in that
- * stream's order, and a block returned by an earlier call may still be read
- * by its queued kernels, so a copy on another stream (or the null stream,
- * which the library's non-blocking streams do not wait for) could overwrite
- * it under them. */
-static int stage_in(const void *arr, size_t bytes, void **dev_out,
-                    int *owned, hipStream_t s)
-{
-    if (plasma_is_device_ptr(arr)) {
-        *dev_out = (void *)arr;
-        *owned = 0;
-        return 0;
-    }
-    *dev_out = plasma_dev_alloc(bytes);
-    if (*dev_out == NULL)
-        return PlasmaErrorOutOfMemory;
-    *owned = 1;
-    return plasma_hip_check(hipMemcpyAsync(*dev_out, arr, bytes,
-                                           hipMemcpyHostToDevice, s),
-                            "hipMemcpyAsync")
-               ? PlasmaErrorInternal : 0;
-}
-
 /* Argument checks of the batched drivers, in the order of their codes:
  * returns -i for an illegal argument i, 1 for the quick return (batch 0),
  * 0 to proceed. */
@@ -168,6 +132,18 @@ static int vbatched16(plasma_context_t *ctx, plasma_enum_t precision,
     return err ? PlasmaErrorInternal : 0;
 }
 
+/* Systems by order, largest first, equal orders by index. */
+static void order_systems(const int *n, int batch, int *order)
+{
+    int start[VBATCH_NMAX + 2] = {0};
+    for (int i = 0; i < batch; i++)
+        start[VBATCH_NMAX - n[i] + 1]++;
+    for (int v = 0; v <= VBATCH_NMAX; v++)
+        start[v + 1] += start[v];
+    for (int i = 0; i < batch; i++)
+        order[start[VBATCH_NMAX - n[i]]++] = i;
+}
+
 static int vbatched(plasma_enum_t precision, plasma_enum_t uplo, int batch,
                     const int *n, void *A, const size_t *aoff, int nrhs,
                     void *B, const size_t *boff, int *info)
@@ -182,31 +158,40 @@ static int vbatched(plasma_enum_t precision, plasma_enum_t uplo, int batch,
     if (args != 0)
         return args < 0 ? args : PlasmaSuccess;
 
-    /* host view of n: the argument check and the order */
+    /* Host view of n (the argument check and the order), and the host
+     * arrays that go to the device, packed for one copy: aoff, boff, n,
+     * order, tickets.  A copy on another stream than the context's could
+     * overwrite a pool block that earlier kernels still read. */
     const size_t nbytes = (size_t)batch * sizeof(int);
     const size_t obytes = (size_t)batch * sizeof(size_t);
-    int *hn = malloc(nbytes);
-    order_t *ord = malloc((size_t)batch * sizeof(order_t));
-    int *hord = malloc(nbytes);
+    const int dev_n = plasma_is_device_ptr(n);
+    const int dev_off = plasma_is_device_ptr(aoff);
+    const int dev_boff = nrhs > 0 && plasma_is_device_ptr(boff);
+    const int dev_info = plasma_is_device_ptr(info);
+    const size_t mbytes = 2 * obytes + 2 * nbytes + 3 * sizeof(int);
     int retval = PlasmaSuccess;
-    void *dn = NULL, *doff = NULL, *dboff = NULL, *dinfo = NULL;
-    int own_n = 0, own_off = 0, own_boff = 0, own_info = 0;
-    void *W = NULL, *dord = NULL, *dticket = NULL;
-    if (hn == NULL || ord == NULL || hord == NULL) {
+    char *meta = NULL;
+    void *W = NULL, *dinfo = NULL;
+    char *host = malloc(mbytes);
+    if (host == NULL) {
         retval = PlasmaErrorOutOfMemory;
         goto done;
     }
-    /* a caller's device array may have been written by work queued on the
-     * library's streams (non-blocking, so the copy below would not wait for
-     * it) */
-    if (plasma_is_device_ptr(n)) {
+    int *hn = (int *)(host + 2 * obytes), *hord = hn + batch;
+    if (dev_n) {
+        /* a caller's device array may have been written by work queued on
+         * the library's streams (non-blocking, so the copy below would not
+         * wait for it) */
         hipStreamSynchronize(ctx->panel_stream);
         hipStreamSynchronize(ctx->stream);
+        if (plasma_hip_check(hipMemcpy(hn, n, nbytes, hipMemcpyDefault),
+                             "hipMemcpy(n)")) {
+            retval = PlasmaErrorInternal;
+            goto done;
+        }
     }
-    if (plasma_hip_check(hipMemcpy(hn, n, nbytes, hipMemcpyDefault),
-                         "hipMemcpy(n)")) {
-        retval = PlasmaErrorInternal;
-        goto done;
+    else {
+        memcpy(hn, n, nbytes);
     }
     int count[3] = {0, 0, 0};
     for (int i = 0; i < batch; i++) {
@@ -216,12 +201,13 @@ static int vbatched(plasma_enum_t precision, plasma_enum_t uplo, int batch,
             goto done;
         }
         count[order_class(hn[i])]++;
-        ord[i].n = hn[i];
-        ord[i].i = i;
     }
-    qsort(ord, batch, sizeof(order_t), by_n_desc);
-    for (int i = 0; i < batch; i++)
-        hord[i] = ord[i].i;
+    order_systems(hn, batch, hord);
+    if (!dev_off)
+        memcpy(host, aoff, obytes);
+    if (nrhs > 0 && !dev_boff)
+        memcpy(host + obytes, boff, obytes);
+    memset(hord + batch, 0, 3 * sizeof(int));
 
     /* one resident grid, each workgroup with its own slab of W */
     const int grid = vbatched_grid(ctx, precision, batch);
@@ -234,47 +220,38 @@ static int vbatched(plasma_enum_t precision, plasma_enum_t uplo, int batch,
                                               ctx->num_cus);
     }
     W = plasma_dev_alloc(wbytes);
-    dord = plasma_dev_alloc(nbytes);
-    dticket = plasma_dev_alloc(3 * sizeof(int));
-    if (W == NULL || dord == NULL || dticket == NULL) {
+    meta = plasma_dev_alloc(mbytes);
+    if (!dev_info)
+        dinfo = plasma_dev_alloc(nbytes);
+    if (W == NULL || meta == NULL || (!dev_info && dinfo == NULL)) {
         retval = PlasmaErrorOutOfMemory;
         goto done;
     }
-    if ((retval = stage_in(n, nbytes, &dn, &own_n, ctx->stream)) != 0 ||
-        (retval = stage_in(aoff, obytes, &doff, &own_off, ctx->stream)) != 0 ||
-        (nrhs > 0 &&
-         (retval = stage_in(boff, obytes, &dboff, &own_boff, ctx->stream)) !=
-             0))
-        goto done;
-    own_info = !plasma_is_device_ptr(info);
-    if (own_info) {
-        dinfo = plasma_dev_alloc(nbytes);
-        if (dinfo == NULL) {
-            retval = PlasmaErrorOutOfMemory;
-            goto done;
-        }
-    }
-    else {
-        dinfo = info;
-    }
     hipStream_t s = ctx->stream;
-    if (plasma_hip_check(hipMemcpyAsync(dord, hord, nbytes,
+    if (plasma_hip_check(hipMemcpyAsync(meta, host, mbytes,
                                         hipMemcpyHostToDevice, s),
-                         "hipMemcpy(order)") ||
-        plasma_kern_fill_int(dticket, 0, 3, s) != 0) {
+                         "hipMemcpyAsync")) {
         retval = PlasmaErrorInternal;
         goto done;
     }
+    const size_t *doff = dev_off ? aoff : (const size_t *)meta;
+    const size_t *dboff = nrhs <= 0  ? NULL
+                          : dev_boff ? boff
+                                     : (const size_t *)(meta + obytes);
+    const int *dn = dev_n ? n : (const int *)(meta + 2 * obytes);
+    int *dord = (int *)(meta + 2 * obytes + nbytes);
+    int *dticket = dord + batch;
+    int *di = dev_info ? info : dinfo;
     if (classes
             ? vbatched16(ctx, precision, uplo == PlasmaUpper, batch, count, dn,
-                         A, doff, W, nrhs, B, dboff, dinfo, dord, dticket)
+                         A, doff, W, nrhs, B, dboff, di, dord, dticket)
             : plasma_kern_vbatched_posv(precision, uplo == PlasmaUpper, batch,
-                                        dn, A, doff, W, nrhs, B, dboff, dinfo,
+                                        dn, A, doff, W, nrhs, B, dboff, di,
                                         dord, dticket, grid, s)) {
         retval = PlasmaErrorInternal;
         goto done;
     }
-    if (own_info &&
+    if (!dev_info &&
         plasma_hip_check(hipMemcpyAsync(info, dinfo, nbytes,
                                         hipMemcpyDeviceToHost, s),
                          "hipMemcpy(info)")) {
@@ -289,16 +266,10 @@ done:
      * (also on the error paths) */
     hipStreamSynchronize(ctx->panel_stream);
     hipStreamSynchronize(ctx->stream);
-    if (own_n) plasma_dev_free(dn);
-    if (own_off) plasma_dev_free(doff);
-    if (own_boff) plasma_dev_free(dboff);
-    if (own_info) plasma_dev_free(dinfo);
-    plasma_dev_free(dticket);
-    plasma_dev_free(dord);
+    plasma_dev_free(dinfo);
+    plasma_dev_free(meta);
     plasma_dev_free(W);
-    free(hord);
-    free(ord);
-    free(hn);
+    free(host);
     return retval;
 }
 
