@@ -62,6 +62,10 @@ int plasma_kern_potrf_diag(plasma_enum_t uplo, plasma_desc_t A, int k,
 int plasma_diag128_ok(plasma_desc_t A);
 int plasma_kern_diag128(plasma_enum_t uplo, plasma_desc_t A, int k, void *inv,
                         int *status, hipStream_t s);
+/* and for complex tiles */
+int plasma_zdiag128_ok(plasma_desc_t A);
+int plasma_kern_zdiag128(plasma_enum_t uplo, plasma_desc_t A, int k,
+                         void *inv, int *status, hipStream_t s);
 
 /* Diagonal tile k factored with only the inverses of its 32 x 32 diagonal
  * blocks written to W_kk (the rest of W_kk is left as it was), for the
