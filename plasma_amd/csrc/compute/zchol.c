@@ -143,6 +143,35 @@ done:
     plasma_dev_free(own_inv);
 }
 
+/* Both sweeps of potrs, each in one launch (kernels/zflowsweep.hip).
+ * Returns 0 when the path does not apply (the per-step sweeps run). */
+static int zflow_sweeps(plasma_enum_t uplo, plasma_desc_t A, plasma_desc_t B,
+                        const void *inv, plasma_sequence_t *sequence,
+                        plasma_request_t *request)
+{
+    if (B.mb != A.mb || !plasma_zflow_sweep_ok(A, B.n))
+        return 0;
+    plasma_context_t *ctx = plasma_context_self();
+    hipStream_t s = ctx->stream;
+    const size_t n = plasma_zflow_sweep_ints(B);
+    int *sync = plasma_dev_alloc(2 * n * sizeof(int));
+    if (sync == NULL)
+        return 0;
+    int *st = plasma_sequence_dstatus(sequence, request);
+    int slot;
+    plasma_prof_begin(s, PlasmaProfSweep, 8.0 * 2.0 * B.m * B.m * B.n, 0,
+                      &slot);
+    if (!issue(plasma_kern_fill_int(sync, 0, (int)(2 * n), s), sequence,
+               request) &&
+        !issue(plasma_kern_zflow_sweep(uplo, 0, A, B, inv, sync, st, s),
+               sequence, request))
+        issue(plasma_kern_zflow_sweep(uplo, 1, A, B, inv, sync + n, st, s),
+              sequence, request);
+    plasma_prof_end(s, slot);
+    plasma_dev_free(sync);
+    return 1;
+}
+
 void plasma_pzpotrs(plasma_enum_t uplo, plasma_desc_t A, plasma_desc_t B,
                     const void *inv, plasma_sequence_t *sequence,
                     plasma_request_t *request)
@@ -166,6 +195,10 @@ void plasma_pzpotrs(plasma_enum_t uplo, plasma_desc_t A, plasma_desc_t B,
             return;
         }
         inv = own_inv;
+    }
+    if (zflow_sweeps(uplo, A, B, inv, sequence, request)) {
+        plasma_dev_free(own_inv);
+        return;
     }
     void *S = plasma_dev_alloc((size_t)B.mb * B.nt * B.nb * es);
     if (S == NULL) {

@@ -152,6 +152,14 @@ size_t plasma_flow_sweep_ints(plasma_desc_t B);
 int plasma_kern_flow_sweep(plasma_enum_t uplo, int backward, plasma_desc_t A,
                            plasma_desc_t B, const void *inv, int *sync,
                            const int *status, hipStream_t s);
+/* The same for complex tiles (L^H backward). */
+#define ZFLOW_SWEEP_NRHS 128
+int plasma_zflow_sweep_ok(plasma_desc_t A, int nrhs);
+size_t plasma_zflow_sweep_ints(plasma_desc_t B);
+int plasma_kern_zflow_sweep(plasma_enum_t uplo, int backward,
+                            plasma_desc_t A, plasma_desc_t B,
+                            const void *inv, int *sync, const int *status,
+                            hipStream_t s);
 
 /*
  * Triangular sweeps of potrs (reference pztrsm.c:113-177 and :43-107).
