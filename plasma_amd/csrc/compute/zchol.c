@@ -8,7 +8,7 @@
  * ConjTrans for lower; ConjTrans then NoTrans for upper).
  *
  * Per step k: the diagonal tile is factored and inverted (W_kk) by one
- * workgroup; the panel P(m) = L(m,k) W_kk^H is one launch of 64 x 64
+ * workgroup; the panel P(m) = L(m,k) W_kk^H is one launch of 32 x 32
  * complex MFMA blocks into a panel buffer; the herk / gemm tasks of the
  * step, L(m,n) -= P(m) P(n)^H, run as two launches (the next column on the
  * lookahead stream, the rest on the main stream, which also copies the
@@ -36,18 +36,28 @@ static double zpotrf_flops(double n)
  * Lookahead of one column on two streams.  Per step k:
  *   panel stream:  wait bulk(k - 2);
  *                  narrow(k): column k's update by step k - 1's panels;
+ *                  record narrow(k);
  *                  diagonal tile k (factor + W_kk); panel(k) into buffer
- *                  k % 2; record factor(k)
- *   main stream:   wait factor(k);
- *                  bulk(k): panels of step k copied into L(m,k), and the
- *                  update of columns k + 2 .. mt-1 by them; record bulk(k)
- * so the diagonal tile and panel of step k + 1 run beside the bulk update
- * of step k.  Races are excluded by construction: column k is written by
+ *                  k % 2
+ *   main stream:   wait narrow(k);
+ *                  bulk(k - 1): panels of step k - 1 copied into L(m,k-1),
+ *                  and the update of columns k + 1 .. mt-1 by them; record
+ *                  bulk(k - 1)
+ * so the diagonal tile and panel of step k run beside the bulk update of
+ * step k - 1.  Races are excluded by construction: column k is written by
  * bulk(j) for j <= k - 2 (all waited for) and by narrow(k); buffer k % 2 is
  * rewritten by panel(k + 2) on the panel stream, after narrow(k + 1) read
- * it there and after the wait for bulk(k).
+ * it there and after the wait for bulk(k).  The bulk update waits for
+ * narrow(k), not just for the panel it reads: side by side they take the
+ * matrix cores from each other, and only the narrow one is urgent.
+ *
+ * Once the whole remaining update is short (plasma_zupdate_short) the steps
+ * run on the panel stream alone, the update of all columns instead of
+ * narrow(k): handing over between the streams costs about 10 us a step, more
+ * than the lookahead saves there.  The first such step waits for the last
+ * bulk update.
  */
-#define ZEV_FACTOR 2
+#define ZEV_NARROW 2
 #define ZEV_BULK 3
 
 void plasma_pzpotrf(plasma_enum_t uplo, plasma_desc_t A, void *inv,
@@ -61,8 +71,8 @@ void plasma_pzpotrf(plasma_enum_t uplo, plasma_desc_t A, void *inv,
     const size_t es = plasma_element_size(A.precision);
     const int mt = A.mt;
     void *own_inv = NULL, *panel[2] = {NULL, NULL};
-    hipEvent_t ev[2 + ZEV_FACTOR + ZEV_BULK];
-    int nev = 0, err = 0;
+    hipEvent_t ev[2 + ZEV_NARROW + ZEV_BULK];
+    int nev = 0, err = 0, serial = 0;
     if (inv == NULL &&
         (inv = own_inv = plasma_dev_alloc(plasma_inv_bytes(A))) == NULL)
         err = PlasmaErrorOutOfMemory;
@@ -80,7 +90,7 @@ void plasma_pzpotrf(plasma_enum_t uplo, plasma_desc_t A, void *inv,
         goto done;
     }
     hipEvent_t ev_fork = ev[0], ev_join = ev[1];
-    hipEvent_t *ev_factor = ev + 2, *ev_bulk = ev + 2 + ZEV_FACTOR;
+    hipEvent_t *ev_narrow = ev + 2, *ev_bulk = ev + 2 + ZEV_NARROW;
 
     hipEventRecord(ev_fork, s0);
     hipStreamWaitEvent(s1, ev_fork, 0);
@@ -88,12 +98,13 @@ void plasma_pzpotrf(plasma_enum_t uplo, plasma_desc_t A, void *inv,
         const double kv = plasma_tile_mview(A, k);
         const double rest = (double)A.m - (double)k * A.mb - kv;
         void *pk = panel[k % 2];
+        const int was_serial = serial;
         int slot;
-        /* panel stream */
-        if (k >= 2)
-            hipStreamWaitEvent(s1, ev_bulk[(k - 2) % ZEV_BULK], 0);
-        if (k >= 1) {
+        serial = plasma_zupdate_short(A, k + 1, mt);
+        if (k >= 1 && !was_serial) {
             const double pv = plasma_tile_mview(A, k - 1);
+            if (k >= 2)
+                hipStreamWaitEvent(s1, ev_bulk[(k - 2) % ZEV_BULK], 0);
             plasma_prof_begin(s1, PlasmaProfUpdate,
                               4.0 * (rest + kv) * (rest + kv + 1) * pv -
                                   4.0 * rest * (rest + 1) * pv,
@@ -102,6 +113,17 @@ void plasma_pzpotrf(plasma_enum_t uplo, plasma_desc_t A, void *inv,
                                             panel[(k - 1) % 2], st, s1),
                         sequence, request);
             plasma_prof_end(s1, slot);
+            hipEventRecord(ev_narrow[k % ZEV_NARROW], s1);
+            hipStreamWaitEvent(s0, ev_narrow[k % ZEV_NARROW], 0);
+            if (!err) {
+                plasma_prof_begin(s0, PlasmaProfUpdate,
+                                  4.0 * rest * (rest + 1) * pv, 0, &slot);
+                err = issue(plasma_kern_zupdate(uplo, A, k - 1, k + 1, mt, 1,
+                                                panel[(k - 1) % 2], st, s0),
+                            sequence, request);
+                plasma_prof_end(s0, slot);
+            }
+            hipEventRecord(ev_bulk[(k - 1) % ZEV_BULK], s0);
         }
         if (!err) {
             plasma_prof_begin(s1, PlasmaProfPotrf, zpotrf_flops(kv), 0,
@@ -117,19 +139,18 @@ void plasma_pzpotrf(plasma_enum_t uplo, plasma_desc_t A, void *inv,
                         sequence, request);
             plasma_prof_end(s1, slot);
         }
-        hipEventRecord(ev_factor[k % ZEV_FACTOR], s1);
-        /* main stream */
-        hipStreamWaitEvent(s0, ev_factor[k % ZEV_FACTOR], 0);
+        if (!serial)
+            continue;
+        if (k >= 1 && !was_serial)
+            hipStreamWaitEvent(s1, ev_bulk[(k - 1) % ZEV_BULK], 0);
         if (!err && k < mt - 1) {
-            const double r2 = rest - plasma_tile_mview(A, k + 1);
-            plasma_prof_begin(s0, PlasmaProfUpdate,
-                              4.0 * r2 * (r2 + 1) * kv, 0, &slot);
-            err = issue(plasma_kern_zupdate(uplo, A, k, k + 2, mt, 1, pk, st,
-                                            s0),
+            plasma_prof_begin(s1, PlasmaProfUpdate,
+                              4.0 * rest * (rest + 1) * kv, 0, &slot);
+            err = issue(plasma_kern_zupdate(uplo, A, k, k + 1, mt, 1, pk, st,
+                                            s1),
                         sequence, request);
-            plasma_prof_end(s0, slot);
+            plasma_prof_end(s1, slot);
         }
-        hipEventRecord(ev_bulk[k % ZEV_BULK], s0);
     }
     hipEventRecord(ev_join, s1);
     hipStreamWaitEvent(s0, ev_join, 0);

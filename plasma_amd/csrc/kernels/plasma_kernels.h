@@ -481,6 +481,9 @@ int plasma_kern_ztrtri_diag(plasma_enum_t uplo, plasma_desc_t A, void *inv,
 int plasma_kern_zpanel(plasma_enum_t uplo, plasma_desc_t A, int k,
                        const void *inv, void *panel_buf, const int *status,
                        hipStream_t s);
+/* Whether the update of columns [n_first, n_end) is so short that it is best
+ * run in the critical chain itself, without lookahead. */
+int plasma_zupdate_short(plasma_desc_t A, int n_first, int n_end);
 int plasma_kern_zupdate(plasma_enum_t uplo, plasma_desc_t A, int k,
                         int n_first, int n_end, int copy,
                         const void *panel_buf, const int *status,

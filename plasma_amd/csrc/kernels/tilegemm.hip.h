@@ -235,6 +235,10 @@ __host__ __device__ __forceinline__ int xcd_grid(int njobs)
 {
     return (njobs + NXCD - 1) / NXCD * NXCD;
 }
+__device__ __forceinline__ int xcd_job(int b, int njobs)
+{
+    return (b % NXCD) * (xcd_grid(njobs) / NXCD) + b / NXCD;
+}
 
 // XU / YU: the decoder's X / Y views have unit row stride (else unit k
 // stride); fixed at compile time so each loader has one code path.  The

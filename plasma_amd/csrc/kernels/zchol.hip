@@ -20,6 +20,7 @@
 // kernels work on L = U^H, reading and writing the stored upper tiles
 // conjugate-transposed, so each algorithm is written once, for L.
 #include "common.hip.h"
+#include "directgemm.hip.h"
 #include "plasma_kernels.h"
 #include "zview.hip.h"
 
@@ -151,7 +152,7 @@ __host__ __device__ __forceinline__ int cdiv(int a, int b)
 }
 
 // ---------------------------------------------------------------------------
-// Block jobs.  A launch is a list of 64 x 64 blocks of output windows; block
+// Block jobs: the per-step sweeps and the residual.  A launch is a list of 64 x 64 blocks of output windows; block
 // b is C = alpha sum_kt X_kt Y_kt (+ C when beta), or a copy of operand 0's
 // X.  The four waves of a workgroup take its 32 x 32 quarters.  ti / tj are
 // the tile indices a decoder needs to find the operands.
@@ -159,7 +160,6 @@ __host__ __device__ __forceinline__ int cdiv(int a, int b)
 template <typename R> struct Job {
     CView<R> C;
     int r0, c0, rows, cols;   // block origin in C and its extent (<= 64)
-    int lower_only;           // only C(r, c) with r >= c
     int copy;                 // C = X of operand 0, no product
     int nk;                   // operand pairs
     int beta;
@@ -194,7 +194,6 @@ __global__ __launch_bounds__(NT) void cjobs_kernel(Dec d, const int *status)
     const int rows = min(32, j.rows - wr), cols = min(32, j.cols - wc);
     if (rows <= 0 || cols <= 0) return;
     const int r0 = j.r0 + wr, c0 = j.c0 + wc;
-    if (j.lower_only && r0 + rows - 1 < c0) return;
     if (j.copy) {
         const Operand<R> o = d.operand(j, 0);
         for (int e = lane; e < 32 * 32; e += 64) {
@@ -210,104 +209,315 @@ __global__ __launch_bounds__(NT) void cjobs_kernel(Dec d, const int *status)
         const Operand<R> o = d.operand(j, kt);
         cprod<R, 2, 2, Dec::PF>(acc, o.X, r0, rows, o.Y, c0, cols, o.K);
     }
-    cstore<R, 2, 2>(acc, j.C, r0, rows, c0, cols, j.alpha, j.beta,
-                    j.lower_only);
+    cstore<R, 2, 2>(acc, j.C, r0, rows, c0, cols, j.alpha, j.beta, 0);
+}
+
+// ---------------------------------------------------------------------------
+// Panel solve and trailing update: C = [C -] X Y^H in blocks of 32 FW x 32 FW,
+// a wave 16 FW x 16 FW of it, as in directgemm.hip.h: operands straight from
+// L2 into a ring of RING 4-deep steps, scalar base addresses, no bounds checks
+// inside (rows past an operand read its last row, their results are not
+// stored).  Y always has contiguous rows (the panel buffer or W); X has, or
+// (upper storage: XU false) contiguous k and is conjugated.  CROW: C has
+// contiguous rows and the product is formed transposed; else C is the
+// conjugated upper tile.
+//
+// Blocks of 32 take 15 us for one column of n = 5001 (K = 128, 8192 cycles of
+// matrix instructions per wave) where blocks of 64 need 28.  Measured, zposv
+// with the bounds-checked block jobs above and with these: n = 900 1608, 1003
+// us; n = 2000 3.42, 2.03 ms; n = 5001 11.1, 7.5 ms (the bulk updates 9.0 ->
+// 3.9 ms, 60% of the matrix rate while diagonal tile and panel run beside
+// them); n = 10000 49.7, 37.2 ms; cposv n = 4000 5.97, 3.81 ms.
+// ---------------------------------------------------------------------------
+template <typename R, int FW, bool CROW, bool ACC, bool XU>
+__device__ __forceinline__ void zproduct(const CView<R> &X, const CView<R> &Y,
+                                         const CView<R> &C, int rows,
+                                         int cols, int K, int lower, int off)
+{
+    constexpr int RING = FW == 1 ? 4 : 3, WT = 16 * FW;
+    typedef typename Mfma<R>::acc_t acc_t;
+    typedef R pair_t __attribute__((ext_vector_type(2)));
+    const int lane = threadIdx.x & 63, l16 = lane & 15, lk = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 3;
+    const int wr = (wave >> 1) * WT, wc = (wave & 1) * WT;
+    rows = dg::uni(rows);
+    cols = dg::uni(cols);
+    K = dg::uni(K);
+    lower = dg::uni(lower);
+    off = dg::uni(off);
+    if (wr >= rows || wc >= cols) return;
+    if (lower && wr + WT - 1 < wc + off) return;
+
+    const DG_GLOBAL char *xp = (const DG_GLOBAL char *)dg::uni(X.p);
+    const DG_GLOBAL char *yp = (const DG_GLOBAL char *)dg::uni(Y.p);
+    DG_GLOBAL char *cp = (DG_GLOBAL char *)dg::uni(C.p);
+    const int ldx = dg::uni(XU ? X.cs : X.rs), ldy = dg::uni(Y.cs);
+    const int ldc = dg::uni(CROW ? C.cs : C.rs);
+    constexpr int ES = (int)sizeof(cx<R>);
+    unsigned xo[FW], yo[FW];
+#pragma unroll
+    for (int i = 0; i < FW; i++) {
+        const int r = min(wr + 16 * i + l16, rows - 1);
+        const int c = min(wc + 16 * i + l16, cols - 1);
+        xo[i] = (XU ? r + lk * ldx : r * ldx + lk) * ES;
+        yo[i] = (c + lk * ldy) * ES;
+    }
+    struct Step {
+        pair_t x[FW], y[FW];
+    };
+    auto load = [&](Step &g, int k) {
+        const DG_GLOBAL char *qx =
+            dg::scalar(xp + (ptrdiff_t)(XU ? k * ldx : k) * ES);
+        const DG_GLOBAL char *qy = dg::scalar(yp + (ptrdiff_t)k * ldy * ES);
+#pragma unroll
+        for (int i = 0; i < FW; i++) {
+            g.x[i] = *(const DG_GLOBAL pair_t *)(qx + xo[i]);
+            g.y[i] = *(const DG_GLOBAL pair_t *)(qy + yo[i]);
+        }
+    };
+    // the last, partial step: k values past K are zero (their lanes read k)
+    auto load_tail = [&](Step &g, int k) {
+        const bool in = k + lk < K;
+        const int h = in ? 0 : lk;
+#pragma unroll
+        for (int i = 0; i < FW; i++) {
+            const DG_GLOBAL char *qx =
+                xp + (ptrdiff_t)(XU ? (k - h) * ldx : k - h) * ES;
+            const DG_GLOBAL char *qy = yp + (ptrdiff_t)(k - h) * ldy * ES;
+            const pair_t x = *(const DG_GLOBAL pair_t *)(qx + xo[i]);
+            const pair_t y = *(const DG_GLOBAL pair_t *)(qy + yo[i]);
+            g.x[i] = in ? x : pair_t{0, 0};
+            g.y[i] = in ? y : pair_t{0, 0};
+        }
+    };
+    // C element (i, j, q): a lane offset and a scalar one
+    constexpr int QS = sizeof(R) == 8 ? 4 : 1;      // Mfma<R>::row per q
+    const unsigned clane = (CROW ? l16 + Mfma<R>::row(lane, 0) * ldc
+                                 : Mfma<R>::row(lane, 0) * ldc + l16) * ES;
+    auto cref = [&](int i, int j, int q) -> DG_GLOBAL pair_t & {
+        const ptrdiff_t o = CROW
+            ? (wr + 16 * i) + (ptrdiff_t)(wc + 16 * j + q * QS) * ldc
+            : (ptrdiff_t)(wr + 16 * i + q * QS) * ldc + (wc + 16 * j);
+        return *(DG_GLOBAL pair_t *)(dg::scalar(cp + o * ES) + clane);
+    };
+    auto crow = [&](int i, int q) {
+        return wr + 16 * i + (CROW ? l16 : Mfma<R>::row(lane, q));
+    };
+    auto ccol = [&](int j, int q) {
+        return wc + 16 * j + (CROW ? Mfma<R>::row(lane, q) : l16);
+    };
+    const bool full = wr + WT <= rows && wc + WT <= cols;
+    pair_t c0[FW][FW][4];
+    if (ACC) {
+#pragma unroll
+        for (int i = 0; i < FW; i++)
+#pragma unroll
+            for (int j = 0; j < FW; j++)
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    if (full || (crow(i, q) < rows && ccol(j, q) < cols))
+                        c0[i][j][q] = cref(i, j, q);
+    }
+    acc_t re[FW][FW], im[FW][FW];
+#pragma unroll
+    for (int i = 0; i < FW; i++)
+#pragma unroll
+        for (int j = 0; j < FW; j++) {
+            re[i][j] = acc_t{0, 0, 0, 0};
+            im[i][j] = acc_t{0, 0, 0, 0};
+        }
+    // x conj(y): Re += xr yr + xi yi, Im += xi yr - xr yi; two passes, so
+    // that consecutive products go to different accumulators
+    auto mma = [](R x, R y, acc_t a) {
+        return CROW ? Mfma<R>::mma(y, x, a) : Mfma<R>::mma(x, y, a);
+    };
+    auto step = [&](const Step &g) {
+#pragma unroll
+        for (int i = 0; i < FW; i++) {
+            const R xr = g.x[i][0], xi = XU ? g.x[i][1] : -g.x[i][1];
+#pragma unroll
+            for (int j = 0; j < FW; j++) {
+                re[i][j] = mma(xr, g.y[j][0], re[i][j]);
+                im[i][j] = mma(xi, g.y[j][0], im[i][j]);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < FW; i++) {
+            const R nr = -g.x[i][0], xi = XU ? g.x[i][1] : -g.x[i][1];
+#pragma unroll
+            for (int j = 0; j < FW; j++) {
+                re[i][j] = mma(xi, g.y[j][1], re[i][j]);
+                im[i][j] = mma(nr, g.y[j][1], im[i][j]);
+            }
+        }
+    };
+    __builtin_amdgcn_sched_barrier(0);
+    Step g[RING];
+    const int nk = K / 4;
+    if (nk >= RING) {
+#pragma unroll
+        for (int u = 0; u < RING; u++) {
+            load(g[u], 4 * u);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        int kc = 0;
+        for (; kc + 2 * RING <= nk; kc += RING) {
+#pragma unroll
+            for (int u = 0; u < RING; u++) {
+                step(g[u]);
+                load(g[u], 4 * (kc + RING + u));
+                // keep the loads this far ahead of their use
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        // the ring, and up to RING - 1 steps still to load
+#pragma unroll
+        for (int u = 0; u < RING; u++) {
+            step(g[u]);
+            if (kc + RING + u < nk) load(g[u], 4 * (kc + RING + u));
+        }
+#pragma unroll
+        for (int u = 0; u < RING - 1; u++)
+            if (kc + RING + u < nk) step(g[u]);
+    }
+    else {
+        for (int kc = 0; kc < nk; kc++) {
+            load(g[0], 4 * kc);
+            step(g[0]);
+        }
+    }
+    if (K % 4 != 0) {
+        load_tail(g[0], 4 * nk);
+        step(g[0]);
+    }
+
+    const bool all = full && !lower;
+#pragma unroll
+    for (int i = 0; i < FW; i++)
+#pragma unroll
+        for (int j = 0; j < FW; j++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int r = crow(i, q), c = ccol(j, q);
+                if (!all && (r >= rows || c >= cols ||
+                             (lower && r < c + off)))
+                    continue;
+                // the conjugated upper tile holds conj(C)
+                pair_t v{re[i][j][q], CROW ? im[i][j][q] : -im[i][j][q]};
+                if (ACC) v = c0[i][j][q] - v;
+                cref(i, j, q) = v;
+            }
+}
+
+// Blocks of 32 FW in a tile side.
+__host__ __device__ __forceinline__ int zblocks(int nb, int fw)
+{
+    return cdiv(nb, 32 * fw);
 }
 
 // Panel of step k: P(m) = L(m,k) W_kk^H for m in (k, mt) into slot m-k-1 of
 // the panel buffer (mb x nb per slot, ld mb): the trsm tasks of
 // pzpotrf.c:47-57 (upper: :90-99), as products with the tile inverse.
-template <typename R> struct PanelDec {
-    // operand steps in flight (cprod): FP64 three, FP32 one
-    static constexpr int PF = (sizeof(R) == 8 ? 3 : 1);
-    plasma_desc_t A;
-    int upper, k, nbr;
-    cx<R> *P;
-    const cx<R> *W;
+template <typename R, bool UPPER>
+__global__ __launch_bounds__(NT, 2) void zpanel_kernel(
+    plasma_desc_t A, int k, cx<R> *P, const cx<R> *W, int njobs,
+    const int *status)
+{
+    if (block_should_stop(status)) return;
+    const int b = tg::xcd_job(blockIdx.x, njobs);
+    if (b >= njobs) return;
+    const int nbr = zblocks(A.mb, 1), per = nbr * nbr;
+    const int m = k + 1 + b / per, blk = b % per;
+    const int r0 = 32 * (blk % nbr), c0 = 32 * (blk / nbr);
+    const int kv = plasma_tile_mview(A, k);
+    const int rows = min(32, plasma_tile_mview(A, m) - r0);
+    const int cols = min(32, kv - c0);
+    if (rows <= 0 || cols <= 0) return;
+    // W is lower triangular: column c of the product needs k <= c
+    zproduct<R, 1, true, false, !UPPER>(
+        lower_cview<R>(A, UPPER, m, k).at(r0, 0),
+        buf_cview((cx<R> *)W + c0, A.mb),
+        buf_cview(P + (size_t)(m - k - 1) * A.mb * A.nb + r0 +
+                      (size_t)c0 * A.mb, A.mb),
+        rows, cols, c0 + cols, 0, 0);
+}
 
-    __device__ bool job(int b, Job<R> &j) const
-    {
-        const int per = nbr * nbr;
-        const int m = k + 1 + b / per, blk = b % per;
-        j.ti = m;
-        j.tj = k;
-        j.C = buf_cview(P + (size_t)(m - k - 1) * A.mb * A.nb, A.mb);
-        job_block(j, 64 * (blk % nbr), 64 * (blk / nbr),
-                  plasma_tile_mview(A, m), plasma_tile_mview(A, k));
-        j.lower_only = 0;
-        j.copy = 0;
-        j.nk = 1;
-        j.alpha = R(1);
-        j.beta = 0;
-        return true;
+// Update of step k: L(m,n) -= P(m) P(n)^H for n >= n_first, n <= m < mt
+// (n_first > k), lower triangle only on diagonal tiles (the herk and gemm
+// tasks of pzpotrf.c:58-78; upper: :100-125).  The first ncopy jobs copy the
+// panels back into L(m,k); the update reads the buffer, not those tiles.
+// One job b, by four waves.
+template <typename R, int FW, bool UPPER>
+__device__ __forceinline__ void zupdate_job(const plasma_desc_t &A, int k,
+                                            int n_first, const cx<R> *P,
+                                            int ncopy, int b)
+{
+    const int nbr = zblocks(A.mb, FW), per = nbr * nbr;
+    const size_t slot = (size_t)A.mb * A.nb;
+    const bool copy = b < ncopy;
+    int m = k + 1 + b / per, n = k;
+    if (!copy) {
+        b -= ncopy;
+        trapezoid_decode(b / per, A.mt, n_first, &m, &n);
     }
-    __device__ Operand<R> operand(const Job<R> &j, int) const
-    {
-        Operand<R> o;
-        o.X = lower_cview<R>(A, upper != 0, j.ti, k);
-        o.Y = herm_of(buf_cview((cx<R> *)W, A.mb));
-        o.K = plasma_tile_mview(A, k);
-        return o;
+    const int blk = b % per, br = blk % nbr, bc = blk / nbr;
+    const int r0 = 32 * FW * br, c0 = 32 * FW * bc;
+    const int rows = min(32 * FW, plasma_tile_mview(A, m) - r0);
+    const int cols = min(32 * FW, plasma_tile_mview(A, n) - c0);
+    if (rows <= 0 || cols <= 0) return;
+    const CView<R> X = buf_cview((cx<R> *)P + (m - k - 1) * slot + r0, A.mb);
+    const CView<R> C = lower_cview<R>(A, UPPER, m, n).at(r0, c0);
+    if (copy) {
+        // along the tile's contiguous index
+        for (int e = threadIdx.x % NT; e < 32 * FW * 32 * FW; e += NT) {
+            const int lo = e % (32 * FW), hi = e / (32 * FW);
+            const int r = UPPER ? hi : lo, c = UPPER ? lo : hi;
+            if (r < rows && c < cols) C.put(r, c, X.raw(r, c0 + c));
+        }
+        return;
     }
-};
+    if (m == n && br < bc) return;
+    zproduct<R, FW, !UPPER, true, true>(
+        X, buf_cview((cx<R> *)P + (n - k - 1) * slot + c0, A.mb), C, rows,
+        cols, plasma_tile_mview(A, k), m == n, c0 - r0);
+}
 
-// Update of step k: L(m,n) -= P(m) P(n)^H for n in [n_first, n_end),
-// n <= m < mt (n_first > k), lower triangle only on diagonal tiles (the
-// herk and gemm tasks of pzpotrf.c:58-78; upper: :100-125).  The first
-// ncopy jobs copy the panels back into L(m,k); the update reads the
-// buffer, not those tiles.
-template <typename R> struct UpdateDec {
-    // operand steps in flight (cprod): FP64 three, FP32 one
-    static constexpr int PF = (sizeof(R) == 8 ? 3 : 1);
-    plasma_desc_t A;
-    int upper, k, nbr, ncopy, n_first;
-    const cx<R> *P;
+// blocks of 32, one workgroup each
+template <typename R, bool UPPER>
+__global__ __launch_bounds__(NT, 2) void zupdate32_kernel(
+    plasma_desc_t A, int k, int n_first, const cx<R> *P, int ncopy, int njobs,
+    const int *status)
+{
+    if (block_should_stop(status)) return;
+    const int b = tg::xcd_job(blockIdx.x, njobs);
+    if (b < njobs)
+        zupdate_job<R, 1, UPPER>(A, k, n_first, P, ncopy, b);
+}
 
-    __device__ bool job(int b, Job<R> &j) const
-    {
-        const int per = nbr * nbr;
-        int m, n;
-        j.lower_only = 0;
-        j.copy = 0;
-        j.nk = 1;
-        j.alpha = R(-1);
-        j.beta = 1;
-        if (b < ncopy) {
-            m = k + 1 + b / per;
-            n = k;
-            j.copy = 1;
-        }
-        else {
-            b -= ncopy;
-            trapezoid_decode(b / per, A.mt, n_first, &m, &n);
-        }
-        const int blk = b % per, br = blk % nbr, bc = blk / nbr;
-        if (!j.copy && m == n) {
-            if (br < bc) return false;
-            j.lower_only = 1;
-        }
-        j.ti = m;
-        j.tj = n;
-        j.C = lower_cview<R>(A, upper != 0, m, n);
-        job_block(j, 64 * br, 64 * bc, plasma_tile_mview(A, m),
-                  plasma_tile_mview(A, n));
-        return true;
-    }
-    __device__ Operand<R> operand(const Job<R> &j, int) const
-    {
-        Operand<R> o;
-        const size_t slot = (size_t)A.mb * A.nb;
-        o.X = buf_cview((cx<R> *)P + (j.ti - k - 1) * slot, A.mb);
-        if (j.copy) {
-            o.Y = o.X;
-            o.K = 0;
-            return o;
-        }
-        o.Y = herm_of(buf_cview((cx<R> *)P + (j.tj - k - 1) * slot, A.mb));
-        o.K = plasma_tile_mview(A, k);
-        return o;
-    }
-};
+// Blocks of 64, two at a time in one resident workgroup of 8 waves, which
+// fills the registers of its CU (FP64: 2 x 216 of 512 per SIMD).  The grid
+// is at most ZU_GRID workgroups, so some CUs stay free for the diagonal tile
+// that runs beside it; it needs a CU's whole LDS and most of its registers
+// and would otherwise wait until the update has nothing left to dispatch (up
+// to 212 us for a tile of 63).
+// The 80 registers left on the other CUs take the 32-wide kernels of the
+// panel and the next column.
+constexpr int ZU_GRID = 240;
+
+template <typename R, bool UPPER>
+__global__ __launch_bounds__(2 * NT, 2) void zupdate64_kernel(
+    plasma_desc_t A, int k, int n_first, const cx<R> *P, int ncopy, int njobs,
+    const int *status)
+{
+    if (block_should_stop(status)) return;
+    const int half = dg::uni(threadIdx.x / NT);
+    const int chunk = tg::xcd_grid(njobs) / tg::NXCD;
+    const int first = blockIdx.x % tg::NXCD * chunk;
+    for (int i = blockIdx.x / tg::NXCD * 2 + half; i < chunk;
+         i += gridDim.x / tg::NXCD * 2)
+        if (first + i < njobs)
+            zupdate_job<R, 2, UPPER>(A, k, n_first, P, ncopy, first + i);
+}
 
 // potrs sweep, diagonal step k: S = W_kk B(k,:) (forward, L Y = B) or
 // W_kk^H B(k,:) (backward, L^H X = Y) into S (mb x B.n, ld mb): the
@@ -330,7 +540,6 @@ template <typename R> struct SweepDiagDec {
         j.C = buf_cview(S + (size_t)jt * B.nb * B.mb, B.mb);
         job_block(j, 64 * (blk % nbr), 64 * (blk / nbr),
                   plasma_tile_mview(B, k), plasma_tile_nview(B, jt));
-        j.lower_only = 0;
         j.copy = 0;
         j.nk = 1;
         j.alpha = R(1);
@@ -378,7 +587,6 @@ template <typename R> struct SweepUpdDec {
         j.C = tile_cview<R>(B, m, jt);
         job_block(j, 64 * (blk % nbr), 64 * (blk / nbr),
                   plasma_tile_mview(B, m), plasma_tile_nview(B, jt));
-        j.lower_only = 0;
         j.nk = 1;
         j.alpha = R(-1);
         j.beta = 1;
@@ -423,7 +631,6 @@ template <typename R> struct ResidualDec {
         j.C = tile_cview<R>(Rd, m, jt);
         job_block(j, 64 * (blk % nbr), 64 * (blk / nbr),
                   plasma_tile_mview(Rd, m), plasma_tile_nview(Rd, jt));
-        j.lower_only = 0;
         j.copy = 0;
         j.nk = A.mt;
         j.alpha = R(-1);
@@ -763,14 +970,27 @@ template <typename R>
 int panel(plasma_enum_t uplo, plasma_desc_t A, int k, const void *inv,
           void *P, const int *status, hipStream_t s)
 {
-    PanelDec<R> d;
-    d.A = A;
-    d.upper = uplo == PlasmaUpper;
-    d.k = k;
-    d.nbr = cdiv(A.mb, 64);
-    d.P = (cx<R> *)P;
-    d.W = (const cx<R> *)inv + (size_t)k * A.mb * A.mb;
-    return launch_jobs<R>(d, (long)(A.mt - k - 1) * d.nbr * d.nbr, status, s);
+    const int nbr = zblocks(A.mb, 1);
+    const long njobs = (long)(A.mt - k - 1) * nbr * nbr;
+    if (njobs <= 0) return 0;
+    if (njobs > 0x7ffffff0L) return PlasmaErrorNotSupported;
+    const cx<R> *W = (const cx<R> *)inv + (size_t)k * A.mb * A.mb;
+    const dim3 grid((unsigned)tg::xcd_grid((int)njobs));
+    if (uplo == PlasmaUpper)
+        hipLaunchKernelGGL((zpanel_kernel<R, true>), grid, dim3(NT), 0, s, A,
+                           k, (cx<R> *)P, W, (int)njobs, status);
+    else
+        hipLaunchKernelGGL((zpanel_kernel<R, false>), grid, dim3(NT), 0, s, A,
+                           k, (cx<R> *)P, W, (int)njobs, status);
+    return done();
+}
+
+// tiles of columns [n_first, n_end): column n holds mt - n of them
+long update_tiles(plasma_desc_t A, int n_first, int n_end)
+{
+    long tiles = 0;
+    for (int n = n_first; n < n_end; n++) tiles += A.mt - n;
+    return tiles;
 }
 
 template <typename R>
@@ -778,20 +998,30 @@ int update(plasma_enum_t uplo, plasma_desc_t A, int k, int n_first,
            int n_end, int copy, const void *P, const int *status,
            hipStream_t s)
 {
-    UpdateDec<R> d;
-    d.A = A;
-    d.upper = uplo == PlasmaUpper;
-    d.k = k;
-    d.n_first = n_first;
-    d.nbr = cdiv(A.mb, 64);
-    d.P = (const cx<R> *)P;
-    const long per = (long)d.nbr * d.nbr;
-    const long rest = (long)A.mt - k - 1;
-    d.ncopy = copy ? (int)(rest * per) : 0;
-    // tiles of columns [n_first, n_end): column n holds mt - n of them
-    long tiles = 0;
-    for (int n = n_first; n < n_end; n++) tiles += A.mt - n;
-    return launch_jobs<R>(d, d.ncopy + tiles * per, status, s);
+    const bool up = uplo == PlasmaUpper;
+    const long tiles = update_tiles(A, n_first, n_end);
+    // one column (the critical chain's) and short updates: blocks of 32
+    const bool w32 = n_end - n_first == 1 ||
+                     plasma_zupdate_short(A, n_first, n_end);
+    const int nbr = zblocks(A.mb, w32 ? 1 : 2);
+    const long per = (long)nbr * nbr;
+    const long ncopy = copy ? ((long)A.mt - k - 1) * per : 0;
+    const long njobs = ncopy + tiles * per;
+    if (njobs <= 0) return 0;
+    if (njobs > 0x7ffffff0L) return PlasmaErrorNotSupported;
+    const int all = tg::xcd_grid((int)njobs);
+    const dim3 grid((unsigned)(w32 ? all : all < ZU_GRID ? all : ZU_GRID));
+    const void *fn =
+        w32 ? (up ? (const void *)zupdate32_kernel<R, true>
+                  : (const void *)zupdate32_kernel<R, false>)
+            : (up ? (const void *)zupdate64_kernel<R, true>
+                  : (const void *)zupdate64_kernel<R, false>);
+    const cx<R> *p = (const cx<R> *)P;
+    int nc = (int)ncopy, nj = (int)njobs;
+    void *args[] = {&A, &k, &n_first, &p, &nc, &nj, &status};
+    return hipLaunchKernel(fn, grid, dim3(w32 ? NT : 2 * NT), args, 0, s) ==
+                   hipSuccess
+               ? 0 : PlasmaErrorInternal;
 }
 
 template <typename R>
@@ -889,6 +1119,13 @@ extern "C" int plasma_kern_zpanel(plasma_enum_t uplo, plasma_desc_t A, int k,
     if (is_z(A)) return panel<double>(uplo, A, k, inv, panel_buf, status, s);
     if (is_c(A)) return panel<float>(uplo, A, k, inv, panel_buf, status, s);
     return PlasmaErrorNotSupported;
+}
+
+// Up to 256 blocks of 64 leave CUs idle: blocks of 32 are done sooner.
+extern "C" int plasma_zupdate_short(plasma_desc_t A, int n_first, int n_end)
+{
+    const long nbr = zblocks(A.mb, 2);
+    return update_tiles(A, n_first, n_end) * nbr * nbr <= 256;
 }
 
 extern "C" int plasma_kern_zupdate(plasma_enum_t uplo, plasma_desc_t A, int k,
