@@ -13,7 +13,8 @@
  *   1. the diagonal-tile inverses W_kk (from the factorization, or formed
  *      for a given factor after a check for a zero diagonal);
  *   2. W = L^{-1} by the forward sweep of the identity (the wide-right-
- *      hand-side sweep: each step one 128 x 128-block MFMA product);
+ *      hand-side sweep; step k on the columns that are not zero, the tile
+ *      columns up to k);
  *   3. Q = W^T W, the triangular Gram product (tiles I >= J of
  *      sum_{K >= I} W(K,I)^T W(K,J), mirrored into a symmetric Q);
  *   4. the uplo triangle of Q into A.
@@ -27,6 +28,39 @@ static int issue(int err, plasma_sequence_t *sequence,
     if (err)
         plasma_request_fail(sequence, request, err);
     return err;
+}
+
+/* W = L^{-1} from W = I: block row k of the sweep is zero to the right of its
+ * diagonal, so step k takes the first k + 1 tile columns only. */
+static void sweep_identity(plasma_enum_t uplo, plasma_desc_t A,
+                           plasma_desc_t W, const void *inv, int *st,
+                           hipStream_t s, plasma_sequence_t *sequence,
+                           plasma_request_t *request)
+{
+    const size_t es = plasma_element_size(W.precision);
+    void *scratch = plasma_dev_alloc((size_t)A.mb * W.nt * W.nb * es);
+    if (scratch == NULL) {
+        plasma_request_fail(sequence, request, PlasmaErrorOutOfMemory);
+        return;
+    }
+    for (int k = 0, err = 0; k < W.mt && !err; k++) {
+        const int cols = imin((k + 1) * W.nb, W.n);
+        const plasma_desc_t Wk = plasma_desc_view(W, 0, 0, W.m, cols);
+        const double nbk = plasma_tile_mview(W, k);
+        int slot;
+        plasma_prof_begin(s, PlasmaProfSweep,
+                          nbk * nbk * cols +
+                              2.0 * nbk * (W.mt - 1 - k) * W.mb * cols,
+                          0, &slot);
+        err = issue(plasma_kern_trsm_diag_left(uplo, 0, A, Wk, k, inv,
+                                               scratch, st, s),
+                    sequence, request) ||
+              issue(plasma_kern_sweep_update(uplo, 0, A, Wk, k, scratch, st,
+                                             s),
+                    sequence, request);
+        plasma_prof_end(s, slot);
+    }
+    plasma_dev_free(scratch);
 }
 
 static void omp_inverse(plasma_enum_t precision, plasma_enum_t uplo,
@@ -103,9 +137,7 @@ static void omp_inverse(plasma_enum_t precision, plasma_enum_t uplo,
     /* 2. W = L^{-1}: the forward sweep (L = U^T for upper storage) of I */
     if (sequence->status == PlasmaSuccess &&
         !issue(plasma_kern_identity(W, st, s), sequence, request))
-        plasma_pxtrsm_left(uplo, uplo == PlasmaUpper ? PlasmaConjTrans
-                                                     : PlasmaNoTrans,
-                           A, W, inv, sequence, request);
+        sweep_identity(uplo, A, W, inv, st, s, sequence, request);
     /* 3. Q = W^T W (W is lower triangular, held in a general descriptor);
      * 4. A's triangle from Q */
     if (sequence->status == PlasmaSuccess &&

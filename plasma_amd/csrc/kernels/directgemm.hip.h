@@ -303,4 +303,21 @@ __global__ __launch_bounds__(NT, 2) void kernel(Decode dec, int njobs,
     run<T, FW, CROW, ACC, XU, YU>(job);
 }
 
+// Block width of the direct kernel for a launch of n128
+// 128 x 128 blocks, in units of 32; 0: the staged kernels.  Up to W_32 of
+// them even 64 x 64 blocks leave most CUs idle; beyond W_64 (two rounds of
+// the chip's workgroup slots) the staged kernels' smaller operand traffic
+// counts.  FP64 solves (nrhs 64 / 10 / 1): n = 500 512 us with the staged
+// kernels alone, 444 with 64 x 64 blocks, 437 with both widths; n = 2049
+// 2186, 1762, 1734 us; n = 8192 12.6, 10.1, 10.0 ms.  W_64 = 512: n = 16384
+// 40.3 ms, 1024: 40.1, 2048: 40.0 (staged alone 44.0); W_32 = 64: n = 8192
+// 10.2 ms.  One launch at n = 8192: panel 28.6 -> 16.8 us beside the bulk
+// update, next column's update (K = 128) 27 -> 12 us.
+constexpr long W_32 = 24, W_64 = 1024;
+
+inline int width(long n128)
+{
+    return n128 <= W_32 ? 1 : n128 <= W_64 ? 2 : 0;
+}
+
 }  // namespace dg

@@ -830,23 +830,6 @@ int launch_panel_blocked(plasma_enum_t uplo, plasma_desc_t A, int k,
     return hipGetLastError() == hipSuccess ? 0 : PlasmaErrorInternal;
 }
 
-// Block width of the direct kernel (directgemm.hip.h) for a launch of n128
-// 128 x 128 blocks, in units of 32; 0: the staged kernels.  Up to DG_32 of
-// them even 64 x 64 blocks leave most CUs idle; beyond DG_64 (two rounds of
-// the chip's workgroup slots) the staged kernels' smaller operand traffic
-// counts.  FP64 solves (nrhs 64 / 10 / 1): n = 500 512 us with the staged
-// kernels alone, 444 with 64 x 64 blocks, 437 with both widths; n = 2049
-// 2186, 1762, 1734 us; n = 8192 12.6, 10.1, 10.0 ms.  DG_64 = 512: n = 16384
-// 40.3 ms, 1024: 40.1, 2048: 40.0 (staged alone 44.0); DG_32 = 64: n = 8192
-// 10.2 ms.  One launch at n = 8192: panel 28.6 -> 16.8 us beside the bulk
-// update, next column's update (K = 128) 27 -> 12 us.
-constexpr long DG_32 = 24, DG_64 = 1024;
-
-int dg_width(long n128)
-{
-    return n128 <= DG_32 ? 1 : n128 <= DG_64 ? 2 : 0;
-}
-
 // The direct kernel over the jobs of a decoder with blocks of 32 FW, `tiles`
 // tiles of mb x mb and ncopy copy jobs.  make(blocks per tile side) builds
 // the decoder.  CL: C has unit row stride also for upper storage (the panel
@@ -881,8 +864,8 @@ int launch_trsm_panel(plasma_enum_t uplo, plasma_desc_t A, int k,
     const bool up = uplo == PlasmaUpper;
     const int bpt = (A.mb + tg::BM - 1) / tg::BM;
     const int n128 = ntiles * bpt * bpt;
-    if (dg_width(n128)) {
-        if (dg_width(n128) == 1)
+    if (dg::width(n128)) {
+        if (dg::width(n128) == 1)
             launch_direct<T, 1, PanelDecode, false, true>(
                 up, ntiles, A.mb, status, s, [&](int bp) {
                     return PanelDecode<T, 32>{A, k, bp, up, pbase, pcols, pcol,
@@ -930,9 +913,9 @@ int launch_trailing_update(plasma_enum_t uplo, plasma_desc_t A, int pbase,
     for (int j = 0; j < copy_cols; j++)
         ncopy += max(A.mt - (pbase + j) - 1, 0);
     const long tiles = nblocks / (bpt * bpt);
-    if (dg_width(nblocks) && nblocks > 0) {
+    if (dg::width(nblocks) && nblocks > 0) {
         const bool up = uplo == PlasmaUpper;
-        if (dg_width(nblocks) == 1)
+        if (dg::width(nblocks) == 1)
             launch_direct<T, 1, UpdateDecode, true, false>(
                 up, tiles, A.mb, status, s, [&](int bp) {
                     return UpdateDecode<T, 32>{A, pbase, pcols, kdepth,
@@ -1245,7 +1228,7 @@ extern "C" int plasma_direct_update_ok(plasma_desc_t A, int n_first, int n_end)
     long ntiles = 0;
     for (int n = n_first; n < n_end; n++) ntiles += A.mt - n;
     const long bpt = (A.mb + tg::BM - 1) / tg::BM;
-    return ntiles > 0 && dg_width(ntiles * bpt * bpt) != 0;
+    return ntiles > 0 && dg::width(ntiles * bpt * bpt) != 0;
 }
 
 extern "C" int plasma_kern_trailing_update(plasma_enum_t uplo,

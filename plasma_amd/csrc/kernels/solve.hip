@@ -11,6 +11,7 @@
 // S back into B(k,:).  Rows of a block row are independent, so both
 // launches split the work into blocks of 64 rows x 32 right-hand sides.
 #include "common.hip.h"
+#include "directgemm.hip.h"
 #include "tilegemm.hip.h"
 #include "plasma_kernels.h"
 
@@ -163,14 +164,20 @@ __global__ __launch_bounds__(NTHREADS) void sweep_update_kernel(
 
 // ---------------------------------------------------------------------------
 // Sweeps with many right-hand sides (B.n >= WIDE_RHS, e.g. the n columns of
-// the Cholesky adjoint): the diagonal product S = op(W_kk) B(k, :) and the
-// update B(m, :) -= op(L) S of one sweep step run as 128 x 128 MFMA block
-// GEMMs (tilegemm.hip.h), one job per (tile row, 128-row block, 128-column
-// block), instead of the 64 x 32 blocks sized for a few dozen columns.
+// the inverse): the diagonal product S = op(W_kk) B(k, :) and the update
+// B(m, :) -= op(L) S of one sweep step run as MFMA block GEMMs, one job per
+// (tile row, block of rows, block of columns), instead of the 64 x 32 blocks
+// sized for a few dozen columns: 128 x 128 blocks through LDS
+// (tilegemm.hip.h), or, for short launches, 32 and 64 wide ones straight
+// from L2 (directgemm.hip.h and its rule).  128 x 128 blocks alone and with
+// the short launches in small ones, FP64: potrs n = 1000, nrhs 1024 1190, 561
+// us; n = 2000, nrhs 2000 2.40, 1.48 ms; inverse (which also leaves out the
+// zero tiles of W) n = 3000 4.05, 2.90 ms, n = 6000 14.2, 9.3 ms.  Below
+// WIDE_RHS the 64 x 32 blocks win: n = 3000, nrhs 300 1262, 1382 us.
 // ---------------------------------------------------------------------------
 constexpr int WIDE_RHS = 1024;
 
-template <typename T>
+template <typename T, int BM = tg::BM>
 struct SweepDecode {
     plasma_desc_t A, B;
     const T *inv;
@@ -180,8 +187,8 @@ struct SweepDecode {
     {
         const int ncb = B.nt * cbpt;
         const int rb = b % bpt, cb = (b / bpt) % ncb, t = b / bpt / ncb;
-        const int tn = cb / cbpt, c0 = (cb % cbpt) * tg::BM;
-        const int r0 = rb * tg::BM;
+        const int tn = cb / cbpt, c0 = (cb % cbpt) * BM;
+        const int r0 = rb * BM;
         const int nv = plasma_tile_nview(B, tn);
         const int kv = plasma_tile_mview(B, k);
         if (c0 >= nv) return false;
@@ -241,17 +248,40 @@ struct SweepDecode {
     }
 };
 
-// One launch of a wide sweep step; ACC/NEG and the X layout (XU: unit row
-// stride) are compile-time in the block GEMM.
+// One launch of a wide sweep step over ntiles tile rows; ACC/NEG and the X
+// layout (XU: unit row stride) are compile-time in the block GEMM.
 template <typename T, bool ACC, bool XU>
-int launch_wide(const SweepDecode<T> &d, int njobs, const int *status,
+int launch_wide(const SweepDecode<T> &d, long ntiles, const int *status,
                 hipStream_t s)
 {
-    if (njobs <= 0) return 0;
-    hipLaunchKernelGGL((tg::kernel<T, true, ACC, ACC, XU, false,
-                                   SweepDecode<T>>),
-                       dim3(tg::xcd_grid(njobs)), dim3(tg::NT), 0, s, d, njobs,
-                       status);
+    auto jobs = [&](int bm, int &bpt, int &cbpt) {
+        bpt = (d.A.mb + bm - 1) / bm;
+        cbpt = (d.B.nb + bm - 1) / bm;
+        return ntiles * bpt * d.B.nt * cbpt;
+    };
+    auto direct = [&](auto fw) {
+        constexpr int FW = decltype(fw)::value, BM = 32 * FW;
+        typedef SweepDecode<T, BM> D;
+        D e{d.A, d.B, d.inv, d.S, d.k, d.backward, d.upper, d.diag, 0, 0,
+            d.mlo};
+        const int n = (int)jobs(BM, e.bpt, e.cbpt);
+        hipLaunchKernelGGL((dg::kernel<T, FW, true, ACC, XU, false, D>),
+                           dim3(tg::xcd_grid(n)), dim3(dg::NT), 0, s, e, n,
+                           status);
+    };
+    SweepDecode<T> e = d;
+    const long n128 = jobs(tg::BM, e.bpt, e.cbpt);
+    if (n128 <= 0) return 0;
+    if (n128 > 0x7ffffff0L) return PlasmaErrorNotSupported;
+    if (dg::width(n128) == 1)
+        direct(std::integral_constant<int, 1>());
+    else if (dg::width(n128) == 2)
+        direct(std::integral_constant<int, 2>());
+    else
+        hipLaunchKernelGGL((tg::kernel<T, true, ACC, ACC, XU, false,
+                                       SweepDecode<T>>),
+                           dim3(tg::xcd_grid((int)n128)), dim3(tg::NT), 0, s,
+                           e, (int)n128, status);
     return hipGetLastError() == hipSuccess ? 0 : PlasmaErrorInternal;
 }
 
@@ -261,13 +291,10 @@ int launch_sweep_diag(int backward, plasma_desc_t A, plasma_desc_t B, int k,
                       hipStream_t s)
 {
     if (B.n >= WIDE_RHS) {
-        const int bpt = (A.mb + tg::BM - 1) / tg::BM;
-        const int cbpt = (B.nb + tg::BM - 1) / tg::BM;
         SweepDecode<T> d{A, B, (const T *)inv, (T *)scratch, k, backward, 0,
-                         1, bpt, cbpt, 0};
-        const int njobs = bpt * B.nt * cbpt;
-        return backward ? launch_wide<T, false, false>(d, njobs, status, s)
-                        : launch_wide<T, false, true>(d, njobs, status, s);
+                         1, 0, 0, 0};
+        return backward ? launch_wide<T, false, false>(d, 1, status, s)
+                        : launch_wide<T, false, true>(d, 1, status, s);
     }
     const int rchunks = (B.mb + SW_BM - 1) / SW_BM;
     const int cchunks = (min(B.nb, B.n) + SW_BN - 1) / SW_BN;
@@ -292,15 +319,12 @@ int launch_sweep_update(plasma_enum_t uplo, int backward, plasma_desc_t A,
         // the update as block GEMMs; sweep_update_kernel below then only
         // copies S into B(k, :)
         const int upper = (uplo == PlasmaUpper);
-        const int bpt = (A.mb + tg::BM - 1) / tg::BM;
-        const int cbpt = (B.nb + tg::BM - 1) / tg::BM;
         SweepDecode<T> d{A, B, nullptr, (T *)scratch, k, backward, upper, 0,
-                         bpt, cbpt, mlo};
-        const int njobs = bpt * B.nt * cbpt * ntiles;
+                         0, 0, mlo};
         // X has unit row stride for forward-lower and backward-upper
         const int err = (backward == upper)
-            ? launch_wide<T, true, true>(d, njobs, status, s)
-            : launch_wide<T, true, false>(d, njobs, status, s);
+            ? launch_wide<T, true, true>(d, ntiles, status, s)
+            : launch_wide<T, true, false>(d, ntiles, status, s);
         if (err) return err;
         ntiles = 0;
     }
