@@ -428,11 +428,14 @@ int launch_zdiag128(plasma_enum_t uplo, plasma_desc_t A, int k, void *inv,
 {
     constexpr size_t lds = zd_lds<R>;
     if (lds > 65536) {
-        static int done = 0;
-        if (!done) {
+        static unsigned long long done = 0;     // a bit per device
+        int dev = 0;
+        (void)hipGetDevice(&dev);
+        const unsigned long long bit = 1ull << (dev & 63);
+        if (!(__atomic_load_n(&done, __ATOMIC_RELAXED) & bit)) {
             (void)hipFuncSetAttribute((const void *)zdiag128_kernel<R>,
                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            done = 1;
+            __atomic_fetch_or(&done, bit, __ATOMIC_RELAXED);
         }
     }
     hipLaunchKernelGGL(zdiag128_kernel<R>, dim3(1), dim3(ZD_NT), lds, s, A,
