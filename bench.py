@@ -580,7 +580,7 @@ def complex_line(bench, n, nrhs, steps, cpu_n, threads):
             "frac_peak": round(fl / (ms * 1e-3) / peak, 4),
             "residual_eps": round(resid(A0, X, B0, 2.0 ** -53 if prec == "z"
                                         else 2.0 ** -24), 4),
-            "roofline": roofline(prof, "cjobs_kernel<UpdateDec> (complex "
+            "roofline": roofline(prof, "zupdate64_kernel (complex "
                                  "herk + gemm, four real MFMA products per "
                                  "complex product)", peak),
             "kernels": classes(prof, 1)}

@@ -42,7 +42,7 @@ int plasma_spotrf_vbatched(plasma_enum_t uplo, int batch, const int *n,
  * (code under hipGraph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  Same arguments, results, info values and error codes as
  * plasma_dposv_vbatched; in addition batch > PLASMA_VBATCH_NOALLOC_MAX
- * returns -2.  Its scratch (the persistent grid's diagonal-block inverses,
+ * returns -2.  Its scratch (the workgroups' slabs of workspace,
  * the order of the systems, the ticket, and staged copies of host n / aoff
  * / boff / info) is one fixed device array per GPU of about 36 MB, reserved
  * when the library loads and kept until the process ends, so it calls no

@@ -1,7 +1,7 @@
 /*
- * batched.c -- SPD solves of many independent systems of uneven order in
- * one persistent launch (plasma_{d,s}posv_vbatched, plasma_{d,s}potrf_
- * vbatched).  No counterpart in the reference, which factors one matrix
+ * batched.c -- SPD solves of many independent systems of uneven order
+ * (plasma_{d,s}posv_vbatched, plasma_{d,s}potrf_vbatched): a persistent
+ * launch per class of orders, or one for all with many right-hand sides.  No counterpart in the reference, which factors one matrix
  * per call (compute/zposv.c); each system follows the same algorithm as
  * the reference's tile factorization of a single tile (core_zpotrf.c) and
  * its triangular solves, with LAPACK's info per system.
@@ -209,7 +209,7 @@ static int vbatched(plasma_enum_t precision, plasma_enum_t uplo, int batch,
         memcpy(host + obytes, boff, obytes);
     memset(hord + batch, 0, 3 * sizeof(int));
 
-    /* one resident grid, each workgroup with its own slab of W */
+    /* resident grids, each workgroup with its own slab of W */
     const int grid = vbatched_grid(ctx, precision, batch);
     const int classes = plasma_vbatched16_ok(nrhs);
     size_t wbytes = (size_t)grid * plasma_kern_vbatched_wslab(precision);

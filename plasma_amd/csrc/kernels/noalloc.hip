@@ -12,7 +12,8 @@
 // what every kernel argument and copy uses.
 //
 // Layout (byte offsets, each region 256-byte aligned):
-//   W      grid slabs of the diagonal-block inverses (FP64)
+//   W      the workgroups' slabs: diagonal-block inverses (FP64), or the
+//          right-hand sides of the class launches, which run in turn
 //   ctrl   ticket, invalid-order flag, counts of the two larger classes of
 //          orders, a ticket per class
 //   n      orders (when the caller's array is on the host)

@@ -10,6 +10,8 @@
 // launch then updates every block row still to be solved from S and copies
 // S back into B(k,:).  Rows of a block row are independent, so both
 // launches split the work into blocks of 64 rows x 32 right-hand sides.
+// With tiles of order <= 128 and up to 128 right-hand sides a sweep is one
+// launch instead (flowsweep.hip).
 #include "common.hip.h"
 #include "directgemm.hip.h"
 #include "tilegemm.hip.h"

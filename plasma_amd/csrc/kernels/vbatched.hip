@@ -23,7 +23,7 @@
 // all right-hand sides together: one wave solves the diagonal block in
 // registers (16 steps), then the waves update the rows above on MFMA.
 // Measured: 1024 FP64 systems of 32 to 512 unknowns 2.71 -> 1.75 ms; 4096 FP32
-// systems of 8 to 128 unknowns 700 -> 245 us (427 of them before the host
+// systems of 8 to 128 unknowns 700 -> 250 us (427 of them before the host
 // side ordered by counting and sent its arrays in one copy).  One 512 x 512
 // FP64 system: 0.72 ms alone, 0.83 ms with one system per CU, of which the
 // products take 0.44 ms (matrix-core floor 0.16; every MFMA needs 1.4 operand

@@ -14,7 +14,7 @@
 // with every lane loading one whole complex element per operand slot.  A
 // complex product carries four times the real one's arithmetic per operand
 // byte, and an FP64 MFMA takes 64 cycles, so the operands come straight from
-// memory (L2) into registers one 4-deep step ahead, without LDS.
+// memory (L2) into registers some 4-deep steps ahead, without LDS.
 //
 // Lower-equivalent convention: for uplo == PlasmaUpper (A = U^H U) the
 // kernels work on L = U^H, reading and writing the stored upper tiles
