@@ -178,8 +178,13 @@ static int k_panel(const group_t *g, int k, void *panel, int pbase,
         ? plasma_kern_trsm_panel_blocked(g->uplo, g->A, k, g->inv, panel,
                                          pbase, g->pcols,
                                          (k - pbase) * g->A.nb, g->st, s)
-        : plasma_kern_trsm_panel(g->uplo, g->A, k, g->inv, panel, pbase,
-                                 g->pcols, (k - pbase) * g->A.nb, g->st, s);
+        : plasma_panel_subst_ok(g->A)
+            ? plasma_kern_panel_subst(g->uplo, g->A, k, g->inv, panel, pbase,
+                                      g->pcols, (k - pbase) * g->A.nb, g->st,
+                                      s)
+            : plasma_kern_trsm_panel(g->uplo, g->A, k, g->inv, panel, pbase,
+                                     g->pcols, (k - pbase) * g->A.nb, g->st,
+                                     s);
     if (!err && split_is_fp16(g->split))
         err = plasma_kern_split16_panel(g->A, k, pbase, g->pcols, panel,
                                         planes_of(g, panel),
@@ -368,14 +373,16 @@ static int pxpotrf_launch(plasma_enum_t uplo, plasma_desc_t A, void *inv,
 {
     plasma_context_t *ctx = plasma_context_self();
     const int gw = imax(1, imin(ctx->group, A.mt));
-    /* Blocked panel solve (diagonal-block inverses only on the critical
-     * path): FP32 tiles too large for the one-pass diagonal kernel, which
-     * forms the whole W_kk (kernels/diagtile.hip; with it the panel is one
-     * product).  In FP64 its panel slows more than the diagonal tile gains
-     * (n = 32768, nb 256: 252.5 -> 281.8 ms), so FP64 keeps the full-inverse
-     * panel product at every tile size. */
+    /* FP32 panels are solved by substitution over blocks (16 columns where
+     * the diagonal tile fits the one-pass kernel, which forms the whole W_kk;
+     * else 32, with only those diagonal blocks of W_kk on the critical path):
+     * the product with the inverse of a whole tile loses accuracy with the
+     * tile's condition (kernels/substpanel.hip), which an FP32 factor cannot
+     * spare.  FP64 takes the product: there the blocked panel slows more than
+     * the diagonal tile gains (n = 32768, nb 256: 252.5 -> 281.8 ms). */
     const int blocked = A.precision == PlasmaRealFloat &&
-                        !plasma_diag128_ok(A) && plasma_panel_blocked_ok(A);
+                        !plasma_panel_subst_ok(A) &&
+                        plasma_panel_blocked_ok(A);
     const int split = use_split(A);
     const int pcols = gw * A.nb;
     /* fp16 terms: the row scales follow the planes of panel buffer 0 */

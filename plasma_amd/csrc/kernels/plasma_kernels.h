@@ -81,6 +81,14 @@ int plasma_kern_trsm_panel_blocked(plasma_enum_t uplo, plasma_desc_t A, int k,
                                    int pcols, int pcol, const int *status,
                                    hipStream_t s);
 
+/* The same for FP32 tiles of order mb <= 128 (plasma_panel_subst_ok) by
+ * 16-column blocks, whose inverses are the diagonal blocks of W_kk. */
+int plasma_panel_subst_ok(plasma_desc_t A);
+int plasma_kern_panel_subst(plasma_enum_t uplo, plasma_desc_t A, int k,
+                            const void *inv, void *panel, int pbase,
+                            int pcols, int pcol, const int *status,
+                            hipStream_t s);
+
 /* Public BLAS-3 (kernels/blas3.hip).  C = alpha op(A) op(B) + beta C on
  * general tile descriptors (views allowed), transa / transb PlasmaNoTrans or
  * (Conj)Trans; tri = PlasmaLower / PlasmaUpper restricts the update to that
