@@ -30,29 +30,28 @@ __device__ __forceinline__ int opaque(int x)
 
 // 1 / sqrt(x) of a pivot, one step at a time (Rsqrt::step<S>, S = 0 ..
 // steps - 1), so that the steps can be placed between the eliminations of
-// the column before: 0 for +inf, NaN for x < 0 or NaN.  The hardware's
-// estimate y0 and one correction with e = 1 - x y0^2: in FP32 (1 ulp before
-// it) to second order, without which the whole column carries the estimate's
-// error (batched systems of order 200 to 512: error of x 3.2e-5 instead of
-// 2.7e-5, at no measurable time); in FP64 (about 2^-24) to third order,
+// the column before: 0 for +inf, NaN for x < 0 or NaN.
+//
+// FP32: the FP64 estimate (measured on 10^6 FP32 arguments: 0.88 2^-24 at
+// most), rounded.  The FP32 estimate takes a subnormal pivot for zero (infinite,
+// and NaN once corrected); with one correction step its rms error is the same
+// (0.50 and 0.49 2^-24), at twice the instructions.  A correction in FP64
+// as well (0.46) made the FP32 batched solver 1.2 % and sposv n = 6000 1 %
+// slower without a smaller error in either.
+//
+// FP64: the estimate y0 and one correction with e = 1 - x y0^2 to third order,
 // (1 - e)^{-1/2}.  The clamp keeps x y0 = 0 (not NaN) for an infinite pivot.
 template <typename T> struct Rsqrt;
 template <> struct Rsqrt<float> {
-    static constexpr int steps = 3;
-    float x, y, e;
+    static constexpr int steps = 2;
+    float x, y;
+    double z;
     template <int S> __device__ __forceinline__ void step()
     {
-        if constexpr (S == 0) y = __builtin_amdgcn_rsqf(x);
-        if constexpr (S == 1)
-            e = __builtin_fmaf(-__builtin_fminf(x, 0x1.fffffep+127f) * y, y,
-                               1.0f);
-        if constexpr (S == 2) y = __builtin_fmaf(0.5f * y, e, y);
+        if constexpr (S == 0) z = __builtin_amdgcn_rsq((double)x);
+        if constexpr (S == 1) y = (float)z;
     }
-    __device__ __forceinline__ void rest()
-    {
-        step<1>();
-        step<2>();
-    }
+    __device__ __forceinline__ void rest() { step<1>(); }
 };
 template <> struct Rsqrt<double> {
     static constexpr int steps = 5;
