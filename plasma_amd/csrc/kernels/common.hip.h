@@ -78,6 +78,18 @@ __device__ __forceinline__ bool block_should_stop(const int *status)
     return s_stop != 0;
 }
 
+// Loads and stores between workgroups of one launch, on different XCDs with an
+// L2 each: they go through to memory and past the caches.
+template <typename T> __device__ __forceinline__ T agent_load(const T *p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ void agent_store(T *p, T v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Tile (m, n) of the lower-equivalent factor, m >= n.
 template <typename T>
 __device__ __forceinline__ View<T> lower_view(const plasma_desc_t &A,

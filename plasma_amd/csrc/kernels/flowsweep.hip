@@ -12,7 +12,9 @@
 //
 // Progress: block rows are handed out by a ticket in the order of their
 // dependences, so a workgroup only ever waits for workgroups that started
-// before it; the first waits for nobody.
+// before it; the first waits for nobody.  A workgroup that finds the status
+// word set publishes its block row unsolved: others may have started before the
+// word was set and wait for it (what they go on to compute is not used).
 //
 // Visibility between workgroups (on different XCDs, with an L2 each): Y is
 // stored and read by relaxed agent-scope atomics, which go through to memory
@@ -104,16 +106,6 @@ __device__ __forceinline__ typename Mfma<T>::acc_t mul_frag(
     return acc;
 }
 
-template <typename T> __device__ __forceinline__ T agent_load(const T *p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <typename T>
-__device__ __forceinline__ void agent_store(T *p, T v)
-{
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // BACK: L^T X = Y.  UPPER: the factor is stored as U = L^T.  sync: a ticket
 // per launch and mt flags per group of right-hand sides, zero on entry.
 template <typename T, bool BACK, bool UPPER>
@@ -127,7 +119,7 @@ __global__ __launch_bounds__(FS_NT) void flow_sweep_kernel(
     __shared__ T sy[2][FS_NB * FS_LD];
     __shared__ int s_ticket;
     if (threadIdx.x == 0) s_ticket = atomicAdd(sync, 1);
-    if (block_should_stop(status)) return;  // and the ticket's barrier
+    const bool stop = block_should_stop(status);    // and the ticket's barrier
     const int ticket = dg::uni(s_ticket);
     const int ngrp = B.nt * gpt;
     const int t = ticket / ngrp, g = ticket % ngrp;
@@ -137,6 +129,10 @@ __global__ __launch_bounds__(FS_NT) void flow_sweep_kernel(
     const int nv = plasma_tile_nview(B, tn) - c0;
     if (nv <= 0) return;                    // an empty group: nobody waits
     int *flags = sync + 1 + (size_t)g * mt;
+    if (stop) {
+        if (threadIdx.x == 0) agent_store(&flags[t], 1);
+        return;
+    }
     const int m = BACK ? mt - 1 - t : t;
     const int mv = plasma_tile_mview(B, m);
     const int lane = threadIdx.x & 63;

@@ -150,7 +150,8 @@ int plasma_direct_update_ok(plasma_desc_t A, int n_first, int n_end);
  * One sweep of potrs in one launch (real tiles of order <= 128 and at most
  * FLOW_SWEEP_NRHS right-hand sides: plasma_flow_sweep_ok): L Y = B forward,
  * L^T X = Y backward, B overwritten.  sync: plasma_flow_sweep_ints(B) ints,
- * zero before the launch.  Up to FLOW_SWEEP_RSOLVE right-hand sides it is
+ * zero before the launch.  The launch ends also when the status word is set
+ * while it runs.  Up to FLOW_SWEEP_RSOLVE right-hand sides it is
  * also the form for a factor that is solved with many times.
  */
 #define FLOW_SWEEP_NRHS 128

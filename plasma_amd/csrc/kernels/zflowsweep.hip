@@ -106,16 +106,6 @@ __device__ __forceinline__ typename Mfma<R>::acc_t mul_half(
     return s;
 }
 
-template <typename R> __device__ __forceinline__ R zagent_load(const R *p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <typename R>
-__device__ __forceinline__ void zagent_store(R *p, R v)
-{
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // BACK: L^H X = Y.  UPPER: the factor is stored as U = L^H.  sync: a ticket
 // per launch and mt flags per group of right-hand sides, zero on entry.
 template <typename R, bool BACK, bool UPPER>
@@ -129,7 +119,7 @@ __global__ __launch_bounds__(ZF_NT) void zflow_sweep_kernel(
     __shared__ R sy[2 * ZF_Y2];
     __shared__ int s_ticket;
     if (threadIdx.x == 0) s_ticket = atomicAdd(sync, 1);
-    if (block_should_stop(status)) return;  // and the ticket's barrier
+    const bool stop = block_should_stop(status);    // and the ticket's barrier
     const int ticket = dg::uni(s_ticket);
     const int ngrp = B.nt * gpt;
     const int t = ticket / ngrp, g = ticket % ngrp;
@@ -139,6 +129,10 @@ __global__ __launch_bounds__(ZF_NT) void zflow_sweep_kernel(
     const int nv = plasma_tile_nview(B, tn) - c0;
     if (nv <= 0) return;                    // an empty group: nobody waits
     int *flags = sync + 1 + (size_t)g * mt;
+    if (stop) {                             // as in the real sweep
+        if (threadIdx.x == 0) agent_store(&flags[t], 1);
+        return;
+    }
     const int m = BACK ? mt - 1 - t : t;
     const int mv = plasma_tile_mview(B, m);
     const int lane = threadIdx.x & 63;
@@ -177,8 +171,8 @@ __global__ __launch_bounds__(ZF_NT) void zflow_sweep_kernel(
             re[u] = im[u] = R(0);
             if (r < kv && c < nv) {
                 const cx<R> *p = Y.p + r + (ptrdiff_t)(c0 + c) * Y.cs;
-                re[u] = zagent_load(&p->re);
-                im[u] = zagent_load(&p->im);
+                re[u] = agent_load(&p->re);
+                im[u] = agent_load(&p->im);
             }
         }
 #pragma unroll
@@ -212,7 +206,7 @@ __global__ __launch_bounds__(ZF_NT) void zflow_sweep_kernel(
     load(f1, 0, 1);
     for (int s = 0; s < t; s++) {
         if (threadIdx.x == 0)
-            while (zagent_load(&flags[s]) == 0) __builtin_amdgcn_s_sleep(1);
+            while (agent_load(&flags[s]) == 0) __builtin_amdgcn_s_sleep(1);
         asm volatile("" ::: "memory");
         __syncthreads();
         fetch(s);
@@ -251,12 +245,12 @@ __global__ __launch_bounds__(ZF_NT) void zflow_sweep_kernel(
 #pragma unroll
         for (int q = 0; q < 4; q++) {
             const int r = row0 + Mfma<R>::row(lane, q);
-            if (r < mv && col < nv) zagent_store(bref(r), p[q]);
+            if (r < mv && col < nv) agent_store(bref(r), p[q]);
         }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (threadIdx.x == 0) zagent_store(&flags[t], 1);
+    if (threadIdx.x == 0) agent_store(&flags[t], 1);
 }
 
 template <typename R>
