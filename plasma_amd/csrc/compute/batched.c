@@ -1,10 +1,11 @@
 /*
  * batched.c -- SPD solves of many independent systems of uneven order
  * (plasma_{d,s}posv_vbatched, plasma_{d,s}potrf_vbatched): a persistent
- * launch per class of orders, or one for all with many right-hand sides.  No counterpart in the reference, which factors one matrix
- * per call (compute/zposv.c); each system follows the same algorithm as
- * the reference's tile factorization of a single tile (core_zpotrf.c) and
- * its triangular solves, with LAPACK's info per system.
+ * launch per class of orders, or one for all with many right-hand sides.  No
+ * counterpart in the reference, which factors one matrix per call
+ * (compute/zposv.c); each system follows the same algorithm as the
+ * reference's tile factorization of a single tile (core_zpotrf.c) and its
+ * triangular solves, with LAPACK's info per system.
  *
  * Layout: system i of order n[i] (0 <= n[i] <= 512) is stored column major
  * at A + aoff[i] with leading dimension n[i]; its right-hand sides at
@@ -113,18 +114,26 @@ static int vbatched16(plasma_context_t *ctx, plasma_enum_t precision,
             err = plasma_hip_check(hipEventCreateWithFlags(
                                        &ev[k], hipEventDisableTiming),
                                    "hipEventCreate");
-        if (!err) {
-            hipEventRecord(ev[0], s0);
-            hipStreamWaitEvent(s1, ev[0], 0);
-        }
+        /* the panel stream's launches read what the main stream is still
+         * copying: without the fork they must not start */
+        if (!err)
+            err = plasma_hip_check(hipEventRecord(ev[0], s0),
+                                   "hipEventRecord") ||
+                  plasma_hip_check(hipStreamWaitEvent(s1, ev[0], 0),
+                                   "hipStreamWaitEvent");
     }
-    if (!err)
+    if (!err) {
         err = plasma_kern_vbatched16(precision, upper, batch, cls, n, A, aoff,
                                      w, nrhs, B, boff, info, order, ticket,
                                      ctx->num_cus, s);
-    if (fork && ev[1] != NULL) {
-        hipEventRecord(ev[1], s1);
-        hipStreamWaitEvent(s0, ev[1], 0);
+        /* without the join the main stream's copy of info would come too
+         * early: an error, which the caller returns after waiting for both
+         * streams */
+        if (fork && (plasma_hip_check(hipEventRecord(ev[1], s1),
+                                      "hipEventRecord") ||
+                     plasma_hip_check(hipStreamWaitEvent(s0, ev[1], 0),
+                                      "hipStreamWaitEvent")))
+            err = 1;
     }
     for (int k = 0; k < 2; k++)
         if (ev[k] != NULL)
