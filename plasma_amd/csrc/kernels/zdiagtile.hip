@@ -55,10 +55,11 @@ constexpr int ztri_row(int b)
     return i;
 }
 
-// LDS (elements): slots, X0, X1, info
+// LDS (elements): slots, X0, X1, an identity block, info
 constexpr int ZD_X0 = ZD_SLOTS * ZD_BLK;
 constexpr int ZD_X1 = ZD_X0 + ZD_BLK;
-constexpr int ZD_INFO = ZD_X1 + ZD_BLK;
+constexpr int ZD_ID = ZD_X1 + ZD_BLK;
+constexpr int ZD_INFO = ZD_ID + ZD_BLK;
 template <typename R> constexpr size_t zd_lds = (ZD_INFO + 1) * sizeof(cx<R>);
 
 __device__ __forceinline__ int at16(int r, int c) { return 16 * c + (r ^ c); }
@@ -66,7 +67,12 @@ __device__ __forceinline__ int at16(int r, int c) { return 16 * c + (r ^ c); }
 // ---------------------------------------------------------------------------
 // The panel in registers (panel16.hip.h in complex arithmetic): dd the
 // diagonal block's rows, p the panel rows.  Column j eliminates column c by
-//     a_c -= a_j conj(l_c),  l_c = lane c's element of the scaled column j.
+//     s_c -= a_j conj(l_c),  l_c = lane c's element of the scaled column j,
+// in sums s that start from zero; the column itself is added when its turn as
+// the pivot column comes, and is read from LDS two columns before that (the
+// identity's rows from a block of their own).  Eliminated in place the column is
+// rounded 2 j times at its own size instead of once: error of the factor of one
+// tile against long double 1.07 u instead of 0.67 u, at the same time.
 // ---------------------------------------------------------------------------
 template <typename R> struct Rows {
     R re[16], im[16];
@@ -86,18 +92,15 @@ template <typename R> struct Rows {
     "v_fmac_f32_dpp " d ", " l ", " m " row_newbcast:" c                      \
     " row_mask:0xf bank_mask:0xf\n\t"
 
-// column C and its pivot x = bcast_C(d.re); columns C and C + 1
-#define Z16_ELIM(T, F, MOV)                                                    \
+// column C; columns C and C + 1
+#define Z16_ELIM(T, F)                                                         \
     template <int C>                                                          \
-    __device__ __forceinline__ void zelim1(Rows<T> &d, Rows<T> &p, T &x,      \
-                                           T lr, T li, T xr, T xi)            \
+    __device__ __forceinline__ void zelim1(Rows<T> &d, Rows<T> &p, T lr,      \
+                                           T li, T xr, T xi)                  \
     {                                                                         \
         asm volatile("s_nop 1\n\t" Z16_COL(F, "%0", "%1", "%2", "%3", "%[c]") \
-                     "s_nop 1\n\t" MOV                                        \
-                     " %4, %0 row_newbcast:%[c] row_mask:0xf "                \
-                     "bank_mask:0xf\n\t"                                      \
                      : "+v"(d.re[C]), "+v"(d.im[C]), "+v"(p.re[C]),           \
-                       "+v"(p.im[C]), "=&v"(x)                                \
+                       "+v"(p.im[C])                                          \
                      : [lr] "v"(lr), [li] "v"(li), [xr] "v"(xr),              \
                        [xi] "v"(xi), [c] "i"(C));                             \
     }                                                                         \
@@ -113,8 +116,8 @@ template <typename R> struct Rows {
                      : [lr] "v"(lr), [li] "v"(li), [xr] "v"(xr),              \
                        [xi] "v"(xi), [c] "i"(C), [c1] "i"(C + 1));            \
     }
-Z16_ELIM(double, Z16_F64, "v_mov_b64_dpp")
-Z16_ELIM(float, Z16_F32, "v_mov_b32_dpp")
+Z16_ELIM(double, Z16_F64)
+Z16_ELIM(float, Z16_F32)
 
 // columns C.. two at a time, one step of the next pivot's 1/sqrt after each
 // group
@@ -125,10 +128,7 @@ template <typename R, int C, int S> struct ZElim {
     {
         constexpr int N = C + 1 < 16 ? 2 : 1;
         if constexpr (C + 1 < 16) zelim2<C>(d, p, lr, li, xr, xi);
-        else if constexpr (C == 15) {
-            R x;
-            zelim1<C>(d, p, x, lr, li, xr, xi);
-        }
+        else if constexpr (C == 15) zelim1<C>(d, p, lr, li, xr, xi);
         if constexpr (S < Rsqrt<R>::steps) {
             next.template step<S>();
             __builtin_amdgcn_sched_barrier(0);
@@ -138,9 +138,24 @@ template <typename R, int C, int S> struct ZElim {
     }
 };
 
+// The original columns of the panel, read some columns ahead: the diagonal
+// block's and the panel rows' element of this lane.
+template <typename R> struct Ahead {
+    static constexpr int N = 2;
+    const cx<R> *ds, *ps;
+    cx<R> d[N], p[N];
+    template <int C> __device__ __forceinline__ void read(int r)
+    {
+        if constexpr (C < 16) {
+            d[C % N] = ds[at16(r, C)];
+            p[C % N] = ps[at16(r, C)];
+        }
+    }
+};
+
 template <typename R, int J> struct ZColumns {
     static __device__ __forceinline__ void run(Rows<R> &d, Rows<R> &p, R &piv,
-                                               R y, int r)
+                                               R y, int r, Ahead<R> &a)
     {
         const R lr = d.re[J] * y, li = d.im[J] * y;
         const R xr = p.re[J] * y, xi = p.im[J] * y;
@@ -150,12 +165,19 @@ template <typename R, int J> struct ZColumns {
         p.im[J] = xi;
         if constexpr (J + 1 < 16) {
             Rsqrt<R> next;
-            zelim1<J + 1>(d, p, next.x, lr, li, xr, xi);
+            zelim1<J + 1>(d, p, lr, li, xr, xi);
+            constexpr int N = (J + 1) % Ahead<R>::N;
+            d.re[J + 1] += a.d[N].re;
+            next.x = row_bcast<J + 1>(d.re[J + 1]);
             next.template step<0>();
+            d.im[J + 1] += a.d[N].im;
+            p.re[J + 1] += a.p[N].re;
+            p.im[J + 1] += a.p[N].im;
+            a.template read<J + 1 + Ahead<R>::N>(r);
             __builtin_amdgcn_sched_barrier(0);
             ZElim<R, J + 2, 1>::run(d, p, lr, li, xr, xi, next);
             piv = (r == J + 1) ? next.x : piv;
-            ZColumns<R, J + 1>::run(d, p, piv, next.y, r);
+            ZColumns<R, J + 1>::run(d, p, piv, next.y, r, a);
         }
     }
 };
@@ -299,6 +321,9 @@ __device__ int factor_zdiag128(const CView<R> &L, const int n,
             sm[(2 * s + h) * ZD_BLK + at16(rr, cc)] = v;
         }
     }
+    if (t < ZD_BLK)
+        sm[ZD_ID + at16(t & 15, t >> 4)] =
+            cx<R>{(t & 15) == t >> 4 ? R(1) : R(0), R(0)};
     if (t == 0) *sinfo = seq_failed(status) ? 1 : 0;
     __syncthreads();
     if (*sinfo) return 0;
@@ -312,29 +337,26 @@ __device__ int factor_zdiag128(const CView<R> &L, const int n,
         // phase A
         if (wave < 2) {
             const int rp = opaque(r16);
-            const cx<R> *ds = sm + ztri(J, J) * ZD_BLK;
             const int i = b - nr;           // identity row block
-            const cx<R> *ps = sm + (b < nr ? ztri(J + 1 + b, J)
-                                           : ztri(J, min(i, J))) * ZD_BLK;
+            Ahead<R> a;
+            a.ds = sm + ztri(J, J) * ZD_BLK;
+            a.ps = sm + (b < nr  ? ztri(J + 1 + b, J) * ZD_BLK
+                         : i < J ? ztri(J, i) * ZD_BLK : ZD_ID);
+            a.template read<0>(rp);
 #pragma unroll
-            for (int c = 0; c < 16; c++) {
-                const cx<R> d = ds[at16(rp, c)], x = ps[at16(rp, c)];
-                dd.re[c] = d.re;
-                dd.im[c] = d.im;
-                p.re[c] = x.re;
-                p.im[c] = x.im;
-            }
-            if (i >= J)
-#pragma unroll
-                for (int c = 0; c < 16; c++) {
-                    p.re[c] = (i == J && c == rp) ? R(1) : R(0);
-                    p.im[c] = R(0);
-                }
+            for (int c = 1; c < 16; c++)
+                dd.re[c] = dd.im[c] = p.re[c] = p.im[c] = R(0);
+            dd.re[0] = a.d[0].re;
+            dd.im[0] = a.d[0].im;
+            p.re[0] = a.p[0].re;
+            p.im[0] = a.p[0].im;
+            a.template read<1>(rp);
+            a.template read<2>(rp);
             Rsqrt<R> first;
             first.x = piv = row_bcast<0>(dd.re[0]);
             first.template step<0>();
             first.rest();
-            ZColumns<R, 0>::run(dd, p, piv, first.y, rp);
+            ZColumns<R, 0>::run(dd, p, piv, first.y, rp, a);
         }
         else if (J > 0) {
             // step K beside the panel: its columns c from J + 1 on (row
