@@ -3,8 +3,9 @@ factor of one tile, where little is subtracted from the matrix (G G^H / n + I).
 A FP64 reference is no better than the library's own results there.
 
 Bounds.  Tile of order 128: an entry is rounded at its own size once for each of
-up to 7 block columns of 16 before its own, and inside that one once (complex):
-with 0.4 u a rounding 0.4 sqrt(4.5) = 0.85 u.  Means over a few matrices each.
+up to 7 block columns of 16 before its own, and inside that one once per column
+(real, 7.5 on average) or once (complex): with 0.4 u a rounding 0.4 sqrt(11) =
+1.3 u and 0.4 sqrt(4.5) = 0.85 u.  Means over a few matrices each.
 """
 import numpy as np
 import pytest
@@ -37,7 +38,8 @@ def _lower(a, uplo):
     return np.tril(a) if uplo == L else np.triu(a).conj().T
 
 
-@pytest.mark.parametrize("prec,limit", [("z", 0.85), ("c", 0.85)])
+@pytest.mark.parametrize("prec,limit", [("d", 1.3), ("s", 1.3), ("z", 0.85),
+                                        ("c", 0.85)])
 @pytest.mark.parametrize("uplo", [L, Up])
 def test_tile(plasma, nb_guard, prec, limit, uplo):
     n = 128
