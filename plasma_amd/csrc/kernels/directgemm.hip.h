@@ -142,8 +142,8 @@ template <typename T, int FW, bool UNIT> struct Operand {
 
 // CROW: C has unit row stride (the product is formed as Y X^T, so that 16
 // consecutive rows of a C column sit in 16 lanes); ACC: C is read, and the
-// product is subtracted from it.
-template <typename T, int FW, bool CROW, bool ACC, bool XU, bool YU>
+// product is subtracted from it, with SEGS by segments of k.
+template <typename T, int FW, bool CROW, bool ACC, bool XU, bool YU, bool SEGS>
 __device__ __forceinline__ void run(tg::Job<T> job)
 {
     constexpr int V = Chunk<T>::V, KC = Chunk<T>::KC, WT = 16 * FW;
@@ -230,7 +230,40 @@ __device__ __forceinline__ void run(tg::Job<T> job)
     // C's loads go first, so that waiting for a chunk never waits for a later
     // load
     __builtin_amdgcn_sched_barrier(0);
+    // The product of SEG chunks (16 k values) is summed by itself and then
+    // subtracted from C (SEGS).  One sum over all K rounds K / 4 times at the
+    // size of that sum, also where C nearly cancels it, as in the trailing blocks
+    // of a kernel (RBF) matrix; one chain that starts from C rounds as often at
+    // the size of C, too often where little is subtracted.  Error of the FP64
+    // factor against long double, n = 1000: RBF, noise 1e-3, 471 u with one sum,
+    // 213 u with a chain, 248 u in segments of 32 and 215 u in segments of 16; G
+    // G^T / n + I 1.6, 4.6, 1.1 and 1.4 u.  The subtraction follows the first
+    // chunk of the next segment, so that it does not wait for the matrix unit:
+    // dposv n = 2049 takes 1327 us with and without segments.
+    constexpr int SEG = 16 / KC;
+    auto chunk = [&](int u, const Regs<T, FW> &x, const Regs<T, FW> &y) {
+        if (!ACC || !SEGS || u % SEG != 0) {
+            step(x, y);
+            return;
+        }
+        acc_t prev[FW][FW];
+#pragma unroll
+        for (int i = 0; i < FW; i++)
+#pragma unroll
+            for (int j = 0; j < FW; j++) {
+                prev[i][j] = acc[i][j];
+                acc[i][j] = acc_t{0, 0, 0, 0};
+            }
+        step(x, y);
+#pragma unroll
+        for (int i = 0; i < FW; i++)
+#pragma unroll
+            for (int j = 0; j < FW; j++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) c0[i][j][q] -= prev[i][j][q];
+    };
     Regs<T, FW> gx[RING], gy[RING];
+    static_assert(RING % SEG == 0, "a segment ends inside the ring");
     if (nk >= RING) {
 #pragma unroll
         for (int u = 0; u < RING; u++) {
@@ -242,7 +275,7 @@ __device__ __forceinline__ void run(tg::Job<T> job)
         for (; kc + 2 * RING <= nk; kc += RING) {
 #pragma unroll
             for (int u = 0; u < RING; u++) {
-                step(gx[u], gy[u]);
+                chunk(u, gx[u], gy[u]);
                 X.load(gx[u], (kc + RING + u) * KC);
                 Y.load(gy[u], (kc + RING + u) * KC);
                 // keep the loads this far ahead of their use
@@ -252,7 +285,7 @@ __device__ __forceinline__ void run(tg::Job<T> job)
         // the ring, and up to RING - 1 chunks still to load
 #pragma unroll
         for (int u = 0; u < RING; u++) {
-            step(gx[u], gy[u]);
+            chunk(u, gx[u], gy[u]);
             if (kc + RING + u < nk) {
                 X.load(gx[u], (kc + RING + u) * KC);
                 Y.load(gy[u], (kc + RING + u) * KC);
@@ -260,7 +293,7 @@ __device__ __forceinline__ void run(tg::Job<T> job)
         }
 #pragma unroll
         for (int u = 0; u < RING - 1; u++)
-            if (kc + RING + u < nk) step(gx[u], gy[u]);
+            if (kc + RING + u < nk) chunk(u, gx[u], gy[u]);
     }
     else {
         for (int kc = 0; kc < nk; kc++) {
@@ -300,7 +333,7 @@ __global__ __launch_bounds__(NT, 2) void kernel(Decode dec, int njobs,
     const int jb = (b % tg::NXCD) * chunk + b / tg::NXCD;
     tg::Job<T> job;
     if (jb >= njobs || !dec(jb, job)) return;
-    run<T, FW, CROW, ACC, XU, YU>(job);
+    run<T, FW, CROW, ACC, XU, YU, Decode::SEGS>(job);
 }
 
 // Block width of the direct kernel for a launch of n128

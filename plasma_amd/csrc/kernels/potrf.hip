@@ -566,6 +566,7 @@ __global__ __launch_bounds__(NT, MINB) void potrf_diag_kernel(
 // for upper storage).
 template <typename T, int BM = tg::BM>
 struct UpdateDecode {
+    static constexpr bool SEGS = true;
     plasma_desc_t A;
     int pbase, pcols, kdepth, ncols, n_first, bpt, upper, ncopy;
     const T *panel;
@@ -632,6 +633,7 @@ struct UpdateDecode {
 // + pcol * mb, column major, ld = mb).
 template <typename T, int BM = tg::BM>
 struct PanelDecode {
+    static constexpr bool SEGS = false;     // nothing is subtracted
     plasma_desc_t A;
     int k, bpt, upper, pbase, pcols, pcol;
     const T *inv;

@@ -181,6 +181,7 @@ constexpr int WIDE_RHS = 1024;
 
 template <typename T, int BM = tg::BM>
 struct SweepDecode {
+    static constexpr bool SEGS = false;
     plasma_desc_t A, B;
     const T *inv;
     T *S;

@@ -1,11 +1,14 @@
 """GPU tests of how often the factorizations round, against long double: the
-factor of one tile, where little is subtracted from the matrix (G G^H / n + I).
-A FP64 reference is no better than the library's own results there.
+factor of one tile, where little is subtracted from the matrix (G G^H / n + I),
+and factors of kernel (RBF) matrices, whose trailing blocks nearly cancel.  A
+FP64 reference is no better than the library's own results there.
 
 Bounds.  Tile of order 128: an entry is rounded at its own size once for each of
 up to 7 block columns of 16 before its own, and inside that one once per column
 (real, 7.5 on average) or once (complex): with 0.4 u a rounding 0.4 sqrt(11) =
-1.3 u and 0.4 sqrt(4.5) = 0.85 u.  Means over a few matrices each.
+1.3 u and 0.4 sqrt(4.5) = 0.85 u.  Kernel matrices: 1.5 times the error of a
+factorization by block columns of 32 in NumPy, which subtracts the product of 32
+columns as a whole.  Means over a few matrices each.
 """
 import numpy as np
 import pytest
@@ -58,3 +61,34 @@ def test_tile(plasma, nb_guard, prec, limit, uplo):
         assert pa.potrf(uplo, n, a, n, prec=prec) == 0
         err.append(_error(_lower(a, uplo), _exact(A)))
     assert np.mean(err) <= limit, err
+
+
+def _rbf(n, seed, noise=1e-3):
+    X = np.random.default_rng(seed).standard_normal((n, 8))
+    D2 = sum((X[:, i, None] - X[None, :, i]) ** 2 for i in range(8))
+    return np.exp(-D2 / 8) + noise * np.eye(n)
+
+
+def _by_32_columns(A):
+    F = A.copy()
+    for j in range(0, len(F), 32):
+        k = j + 32
+        F[j:k, j:k] = np.linalg.cholesky(F[j:k, j:k])
+        F[k:, j:k] = np.linalg.solve(F[j:k, j:k], F[k:, j:k].T).T
+        F[k:, k:] -= F[k:, j:k] @ F[k:, j:k].T
+    return np.tril(F)
+
+
+@pytest.mark.parametrize("uplo", [L, Up])
+def test_posv_kernel_matrix(plasma, nb_guard, uplo):
+    n = 512
+    pa.set_param(pa.PlasmaNb, 128)
+    err, lim = [], []
+    for seed in range(3):
+        A = _rbf(n, seed)
+        ref = _exact(A)
+        a = np.asfortranarray(A)
+        assert pa.potrf(uplo, n, a, n) == 0
+        err.append(_error(_lower(a, uplo), ref))
+        lim.append(_error(_by_32_columns(A), ref))
+    assert np.mean(err) <= 1.5 * np.mean(lim), (err, lim)
