@@ -9,10 +9,10 @@
 //
 // Left-looking by block columns J of 16, the matrix in place in global memory
 // (L2), only the block column in LDS:
-//   1. the waves form A(:, J) - L(:, <J) L(J, <J)^T by strips of 16 rows on
-//      MFMA, operands straight from L2 (the matrix is read about n / 96 times
-//      and written once; a right-looking update would also write it that
-//      often), and put the blocks into LDS;
+//   1. the waves put A(:, J) into LDS by strips of 16 rows and subtract
+//      L(:, <J) L(J, <J)^T from it on MFMA, operands straight from L2 (the
+//      matrix is read about n / 96 times and written once; a right-looking
+//      update would also write it that often);
 //   2. every wave eliminates the 16 columns for up to 64 of its rows
 //      (panel16.hip.h; each repeats the diagonal block, so the pivots need no
 //      exchange) and stores them.
@@ -22,7 +22,7 @@
 // factorization has succeeded.  L^T X = Y then goes backwards by 16 rows for
 // all right-hand sides together: one wave solves the diagonal block in
 // registers (16 steps), then the waves update the rows above on MFMA.
-// Measured: 1024 FP64 systems of 32 to 512 unknowns 2.71 -> 1.75 ms; 4096 FP32
+// Measured: 1024 FP64 systems of 32 to 512 unknowns 2.71 -> 1.80 ms; 4096 FP32
 // systems of 8 to 128 unknowns 700 -> 250 us (427 of them before the host
 // side ordered by counting and sent its arrays in one copy).  One 512 x 512
 // FP64 system: 0.72 ms alone, 0.83 ms with one system per CU, of which the
@@ -49,15 +49,32 @@ __device__ __forceinline__ int opaque_s(int x)
     return x;
 }
 
-// acc[g] += (rows of strip g) (rows of block row J)^T over columns 0 .. j0-1,
-// more chunks in flight the fewer strips share a wave's registers.
-template <typename T, int CNT, bool UNIT>
+// (block of strip g in LDS) -= (rows of strip g) (rows of block row J)^T over
+// columns 0 .. j0-1, more chunks in flight the fewer strips share a wave's
+// registers.
+//
+// The product of 32 columns at a time is summed by itself and then subtracted
+// from the block.  One sum over all columns rounds j0 / 4 times at the size of
+// that sum: what is left of A below it is far smaller in a kernel (RBF) matrix
+// (noise 1e-3, error of the FP64 factor against long double with one sum and
+// with this: n = 128 17 and 12.5 u, 256 61 and 33 u, 512 239 and 91 u); one chain
+// that starts from the block rounds as often at the block's size, and that is
+// too often where little is subtracted (G G^T / n + I).  It costs the LDS traffic:
+// 1024 FP64 systems of 32 to 512 unknowns 1.77 -> 1.80 ms; FP32, which summed 32
+// columns apart before but added them up, 4096 systems of 8 to 128 unknowns 251 ->
+// 246 us.  Sums of 64 columns: 137 u at n = 512, and slower.  Adding in LDS by its
+// FP64 atomics: 1.85 ms.
+// The blocks are at `own` and every STRIDE elements after it, the last one at
+// `last`.
+template <typename T, int CNT, bool UNIT, int STRIDE>
 __device__ __forceinline__ void strip_products(
-    typename Mfma<T>::acc_t (&acc)[4], const dg::Operand<T, 1, UNIT> (&op)[4],
+    T *own, T *last, const dg::Operand<T, 1, UNIT> (&op)[4],
     const dg::Operand<T, 1, UNIT> &bop, int j0)
 {
     constexpr int KC = dg::Chunk<T>::KC, V = dg::Chunk<T>::V;
     constexpr int R = CNT <= 2 ? 4 : 2;
+    constexpr int SEG = 32 / KC;        // chunks summed by themselves
+    typename Mfma<T>::acc_t acc[CNT];
     dg::Regs<T, 1> x[R][CNT], b[R];
     // j0 is a multiple of 16, i.e. of KC, and positive; a chunk past the end
     // reads the last one again
@@ -68,51 +85,52 @@ __device__ __forceinline__ void strip_products(
         for (int g = 0; g < CNT; g++) op[g].load(x[u][g], kc);
         __builtin_amdgcn_sched_barrier(0);
     };
-    // FP32 sums two chunks (32 columns) on their own before they meet the
-    // rest: one chain over all j0 terms rounds j0 / 4 times at the size of
-    // the whole sum (4096 systems of order <= 128: error of x 1.0e-5, this way
-    // 8.2e-6).  FP64 has no registers to spare for it.
-    constexpr bool PART = sizeof(T) == 4;
-    typename Mfma<T>::acc_t part[CNT];
     auto clear = [&]() {
 #pragma unroll
         for (int g = 0; g < CNT; g++)
-            part[g] = typename Mfma<T>::acc_t{0, 0, 0, 0};
+            acc[g] = typename Mfma<T>::acc_t{0, 0, 0, 0};
     };
-    auto add = [&]() {
+    auto flush = [&]() {
+        const int l = opaque(threadIdx.x & 63);
+        const int o = Mfma<T>::row(l, 0) * VN_LD + (l & 15);
+        constexpr int QS = (sizeof(T) == 8 ? 4 : 1) * VN_LD;
 #pragma unroll
-        for (int g = 0; g < CNT; g++)
+        for (int g = 0; g < CNT; g++) {
+            T *blk = (g + 1 < CNT ? own + g * STRIDE : last) + o;
 #pragma unroll
-            for (int e = 0; e < 4; e++) acc[g][e] += part[g][e];
+            for (int e = 0; e < 4; e++) blk[e * QS] -= acc[g][e];
+        }
+        clear();
     };
     auto step = [&](int u) {
 #pragma unroll
         for (int v = 0; v < V; v++)
 #pragma unroll
-            for (int g = 0; g < CNT; g++) {
-                typename Mfma<T>::acc_t &to = PART ? part[g] : acc[g];
-                to = Mfma<T>::mma(b[u].v[0][v], x[u][g].v[0][v], to);
-            }
+            for (int g = 0; g < CNT; g++)
+                acc[g] = Mfma<T>::mma(b[u].v[0][v], x[u][g].v[0][v], acc[g]);
     };
     const int nk = j0 / KC;
 #pragma unroll
     for (int u = 0; u < R; u++) load(u, u);
+    clear();
+    constexpr int N = R > SEG ? R : SEG;        // chunks per round
     int i = 0;
-    for (; i + R <= nk; i += R) {
+    for (; i + N <= nk; i += N) {
 #pragma unroll
-        for (int u = 0; u < R; u++) {
-            if (PART && u % 2 == 0) clear();
-            step(u);
-            load(u, i + R + u);
-            if (PART && u % 2 == 1) add();
+        for (int u = 0; u < N; u++) {
+            step(u % R);
+            load(u % R, i + R + u);
+            if ((u + 1) % SEG == 0) flush();
         }
     }
 #pragma unroll
-    for (int u = 0; u < R - 1; u++) {
-        if (PART && u % 2 == 0) clear();
-        if (i + u < nk) step(u);
-        if (PART && (u % 2 == 1 || u == R - 2)) add();
+    for (int u = 0; u < N - 1; u++) {
+        if (i + u >= nk) break;
+        step(u % R);
+        if (u + R < N - 1) load(u % R, i + R + u);
+        if ((u + 1) % SEG == 0) flush();
     }
+    if (nk % SEG != 0) flush();
 }
 
 // x in lane i of a 16-lane row: the equations K, K - 1, .. of L^T x = t with
@@ -180,26 +198,7 @@ __global__ __launch_bounds__(64 * NW, 4) void vbatched16_kernel(
                 return g < cnt ? wave + NW * g : -1;
             };
             const int all = cnt + diag;             // 5 only at J = 0
-            acc_t acc[4];
-#pragma unroll
-            for (int g = 0; g < 4; g++) acc[g] = acc_t{0, 0, 0, 0};
-            if (J > 0 && all > 0) {
-                dg::Operand<T, 1, UNIT> op[4], bop;
-                bop.init(L, j0, n);
-#pragma unroll
-                for (int g = 0; g < 4; g++) {
-                    const int q = strip(g);
-                    if (q == ns)     op[g].init(Y, 0, VN_RHS);
-                    else if (q >= 0) op[g].init(L, j0 + 16 + 16 * q, n);
-                    else             op[g] = bop;
-                }
-                if (all == 1)      strip_products<T, 1, UNIT>(acc, op, bop, j0);
-                else if (all == 2) strip_products<T, 2, UNIT>(acc, op, bop, j0);
-                else if (all == 3) strip_products<T, 3, UNIT>(acc, op, bop, j0);
-                else               strip_products<T, 4, UNIT>(acc, op, bop, j0);
-            }
-            // the blocks, into LDS: A minus the product; padding is zero, on
-            // the diagonal one
+            // the blocks of A into LDS; padding is zero, on the diagonal one
             // (all loads at clamped addresses before the first use)
             const int l1 = opaque(lane), r1 = l1 & 15, n1 = opaque_s(n);
 #pragma unroll
@@ -235,13 +234,45 @@ __global__ __launch_bounds__(64 * NW, 4) void vbatched16_kernel(
                         // inside: a row of the matrix or a right-hand side (row
                         // n1 here), columns up to the diagonal
                         const int c = Mfma<T>::row(l1, e), col = j0 + c;
-                        const T sum = g < 4 ? acc[g < 4 ? g : 0][e] : T(0);
                         const T pad = (q < 0 && r1 == c) ? T(1) : T(0);
                         const bool in = col < n1 && col <= row &&
                                         row < (q == ns ? n1 + 1 : n1);
-                        blk[c * VN_LD + r1] = in ? av[g - g0][e] - sum : pad;
+                        blk[c * VN_LD + r1] = in ? av[g - g0][e] : pad;
                     }
+                }
             }
+            // minus the products, each wave in its own blocks
+            if (J > 0 && all > 0) {
+                dg::Operand<T, 1, UNIT> op[4], bop;
+                bop.init(L, j0, n);
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    const int q = strip(g);
+                    if (q == ns)     op[g].init(Y, 0, VN_RHS);
+                    else if (q >= 0) op[g].init(L, j0 + 16 + 16 * q, n);
+                    else             op[g] = bop;
+                }
+                constexpr int ST = NW * VN_BLK;
+                T *own = sblk + (wave + 1) * VN_BLK;
+                T *last = diag ? sblk : own + (all - 1) * ST;
+                if (all == 1)
+                    strip_products<T, 1, UNIT, ST>(own, last, op, bop, j0);
+                else if (all == 2)
+                    strip_products<T, 2, UNIT, ST>(own, last, op, bop, j0);
+                else if (all == 3)
+                    strip_products<T, 3, UNIT, ST>(own, last, op, bop, j0);
+                else
+                    strip_products<T, 4, UNIT, ST>(own, last, op, bop, j0);
+                // the padding of a last, partial block column again
+                if (diag && j0 + 16 > n) {
+                    const int l0 = opaque(lane), r0 = l0 & 15;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const int c = Mfma<T>::row(l0, e);
+                        if (j0 + max(r0, c) >= n)
+                            sblk[c * VN_LD + r0] = r0 == c ? T(1) : T(0);
+                    }
+                }
             }
             __syncthreads();
 

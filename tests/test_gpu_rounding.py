@@ -92,3 +92,25 @@ def test_posv_kernel_matrix(plasma, nb_guard, uplo):
         err.append(_error(_lower(a, uplo), ref))
         lim.append(_error(_by_32_columns(A), ref))
     assert np.mean(err) <= 1.5 * np.mean(lim), (err, lim)
+
+
+@pytest.mark.parametrize("uplo", [L, Up])
+@pytest.mark.parametrize("n", [128, 250, 400])
+def test_batched_kernel_matrix(plasma, uplo, n):
+    import torch
+    mats = [_rbf(n, seed) for seed in range(4)]
+    order = np.full(4, n, dtype=np.int32)
+    off = (np.arange(4) * n * n).astype(np.uint64)
+    info = np.full(4, -7, dtype=np.int32)
+    d = torch.from_numpy(np.concatenate([A.ravel() for A in mats])).cuda()
+    torch.cuda.synchronize()
+    assert pa.load().plasma_dpotrf_vbatched(
+        uplo, 4, order.ctypes.data, d.data_ptr(), off.ctypes.data,
+        info.ctypes.data) == 0
+    assert not info.any()
+    err, lim = [], []
+    for A, a in zip(mats, d.cpu().numpy().reshape(4, n, n)):
+        ref = _exact(A)
+        err.append(_error(_lower(a.T, uplo), ref))
+        lim.append(_error(_by_32_columns(A), ref))
+    assert np.mean(err) <= 1.5 * np.mean(lim), (err, lim)
