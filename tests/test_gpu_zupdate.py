@@ -4,7 +4,7 @@ no multiple of the 32 and 64 wide blocks, K that is no multiple of 4 or below
 update moves from its own stream (blocks of 64) to the panel's (blocks of 32).
 
 Bound: the relative error of the factor of a well-conditioned matrix is a
-small multiple of sqrt(n) u; 8 n u is used.
+small multiple of sqrt(n) u; 4 sqrt(n) u is used.
 """
 import numpy as np
 import pytest
@@ -35,5 +35,6 @@ def test_factor(plasma, nb_guard, prec, uplo, n, nb):
     ref = np.linalg.cholesky(A.astype(np.complex128))
     got = np.tril(a) if uplo == L else np.triu(a).conj().T
     err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
-    assert err <= 8 * n * (U.EPS64 if prec == "z" else U.EPS32), err
+    assert err <= 4 * np.sqrt(n) * (U.EPS64 if prec == "z"
+                                    else U.EPS32), err
     assert not np.any(np.triu(a, 1) if uplo == L else np.tril(a, -1))
