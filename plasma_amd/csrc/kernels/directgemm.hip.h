@@ -236,8 +236,8 @@ __device__ __forceinline__ void run(tg::Job<T> job)
     // of a kernel (RBF) matrix; one chain that starts from C rounds as often at
     // the size of C, too often where little is subtracted.  Error of the FP64
     // factor against long double, n = 1000: RBF, noise 1e-3, 471 u with one sum,
-    // 213 u with a chain, 248 u in segments of 32 and 215 u in segments of 16; G
-    // G^T / n + I 1.6, 4.6, 1.1 and 1.4 u.  The subtraction follows the first
+    // 213 u with a chain, 248 u in segments of 32 and 215 u in segments of 16; for
+    // G G^T / n + I 1.6, 4.6, 1.1 and 1.4 u.  The subtraction follows the first
     // chunk of the next segment, so that it does not wait for the matrix unit:
     // dposv n = 2049 takes 1327 us with and without segments.
     constexpr int SEG = 16 / KC;

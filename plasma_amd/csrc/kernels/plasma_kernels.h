@@ -271,14 +271,17 @@ int plasma_kern_ssweep(plasma_enum_t uplo, int backward, plasma_desc_t A,
  * plasma_noalloc_setup (called by plasma_init with the device current);
  * plasma_noalloc_regions hands out its parts.  plasma_kern_vbatched_order
  * writes the systems largest order first into `order`, zeroes the ticket
- * ctrl[0] and sets ctrl[1] when an order is outside [0, 512]; n, order and
- * ctrl are device memory, batch <= PLASMA_VBATCH_NOALLOC_MAX.
+ * ctrl[0], sets ctrl[1] when an order is outside [0, 512], counts the orders
+ * above 256 and above 128 into ctrl[2] and ctrl[3] and zeroes a ticket per class
+ * of orders, ctrl[4 .. 6]; n, order and ctrl are device memory, batch <=
+ * PLASMA_VBATCH_NOALLOC_MAX.
  */
 typedef struct {
     void *W;                 /* grid_max slabs of wslab_bytes */
     size_t wslab_bytes;
     int grid_max;
-    int *ctrl;               /* [0] ticket, [1] invalid-order flag */
+    int *ctrl;               /* 7 words: ticket, invalid-order flag, the
+                                counts and tickets of the classes */
     int *n, *order, *info;   /* PLASMA_VBATCH_NOALLOC_MAX entries each */
     size_t *aoff, *boff;
     size_t bytes;            /* the whole array */

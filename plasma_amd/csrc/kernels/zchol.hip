@@ -152,10 +152,11 @@ __host__ __device__ __forceinline__ int cdiv(int a, int b)
 }
 
 // ---------------------------------------------------------------------------
-// Block jobs: the per-step sweeps and the residual.  A launch is a list of 64 x 64 blocks of output windows; block
-// b is C = alpha sum_kt X_kt Y_kt (+ C when beta), or a copy of operand 0's
-// X.  The four waves of a workgroup take its 32 x 32 quarters.  ti / tj are
-// the tile indices a decoder needs to find the operands.
+// Block jobs: the per-step sweeps and the residual.  A launch is a list of
+// 64 x 64 blocks of output windows; block b is C = alpha sum_kt X_kt Y_kt
+// (+ C when beta), or a copy of operand 0's X.  The four waves of a workgroup
+// take its 32 x 32 quarters.  ti / tj are the tile indices a decoder needs to
+// find the operands.
 // ---------------------------------------------------------------------------
 template <typename R> struct Job {
     CView<R> C;

@@ -157,7 +157,8 @@ __global__ __launch_bounds__(ZF_NT) void zflow_sweep_kernel(
                              plasma_tile_mview(B, k), h);
         }
     };
-    // -Y_k into sy (Y2 negated where X is conjugated); rows and right-hand sides past the end are zero
+    // -Y_k into sy (Y2 negated where X is conjugated); rows and right-hand
+    // sides past the end are zero
     auto fetch = [&](int s) {
         const int k = BACK ? mt - 1 - s : s;
         const CView<R> Y = tile_cview<R>(B, k, tn);
