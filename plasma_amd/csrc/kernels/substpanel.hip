@@ -32,6 +32,7 @@
 // kernel the same took 9.2 us: 1200 instructions, 4 us, before the barrier.
 #include "common.hip.h"
 #include "directgemm.hip.h"
+#include "paneltiles.h"
 #include "plasma_kernels.h"
 
 namespace {
@@ -45,18 +46,15 @@ __host__ __device__ constexpr int sp_tri(int i, int j)
     return i * (i + 1) / 2 + j;
 }
 
-// What the kernel needs to know of the descriptor, worked out on the host: the
-// tile arithmetic of a descriptor is some hundred instructions, more than the
-// rest of what precedes the loads.
+// What the kernel needs to know of the descriptor, worked out on the host
+// (paneltiles.h).
 struct Panel {
+    const float *A;             // the matrix
     const float *L, *W;         // L_kk, W_kk
-    const float *A0, *A1;       // A(k+1,k), and the last tile of the column
-    ptrdiff_t step, step2;      // first and second difference of the addresses
-                                // of the tiles before the last one, elements
+    plasma_panel_tiles_t tiles; // A(m,k), m > k
     float *P;                   // solved panel of tile k + 1
     ptrdiff_t pstep;            // from one tile's panel to the next
-    int ldl, lda, lda1, ldp;
-    int nb, rows1, ntiles;      // tile order, rows of the last tile, tiles
+    int ldl, ldp, nb;           // nb: tile order
     const int *status;
 };
 
@@ -73,20 +71,17 @@ __global__ __launch_bounds__(SP_NT, 2) void panel_subst_kernel(Panel g)
     const int g4 = 4 * (lane >> 4);
     const int wave = dg::uni(t >> 6);
     const int m = blockIdx.x;
-    const bool last = m == g.ntiles - 1;
+    const bool last = m == g.tiles.ntiles - 1;
     const int nb = FULL ? 16 * BLKS : g.nb;
-    const int mv = last ? g.rows1 : nb;
+    const int mv = last ? g.tiles.rows_last : nb;
     const int row0 = blockIdx.y * SP_ROWS;
     if (row0 >= mv) return;
     // read beside the blocks: set, nothing is solved
     const int stop = t == 0 ? __atomic_load_n(g.status, __ATOMIC_RELAXED) : 0;
     const int row = row0 + 16 * wave + l16;
     const DG_GLOBAL float *ap =
-        (const DG_GLOBAL float *)(last ? g.A1
-                                       : g.A0 + m * g.step +
-                                             m * (ptrdiff_t)(m - 1) / 2 *
-                                                 g.step2);
-    const int lda = last ? g.lda1 : g.lda;
+        (const DG_GLOBAL float *)(g.A + plasma_panel_tile(&g.tiles, m));
+    const int lda = last ? g.tiles.ld_last : g.tiles.ld;
 
     // Rows r0 + lane % 16, columns c0 + 4 (lane / 16) + 0 .. 3 of a window of
     // `rows` rows and nb columns; element (r, c) at p[r + c ld] (UNIT) or
@@ -251,42 +246,30 @@ extern "C" int plasma_kern_panel_subst(plasma_enum_t uplo, plasma_desc_t A,
     if (!plasma_panel_subst_ok(A)) return PlasmaErrorNotSupported;
     if (A.mt - k - 1 <= 0) return 0;
     const bool up = uplo == PlasmaUpper, small = A.mb <= 64;
-    // tile (m, k) of the lower-equivalent factor
-    auto tile = [&](int m) {
-        return (const float *)(up ? plasma_tile_addr(A, k, m)
-                                  : plasma_tile_addr(A, m, k));
-    };
     const size_t mb = A.mb;
     Panel g;
-    g.ntiles = A.mt - k - 1;
-    g.L = tile(k);
+    g.A = (const float *)A.matrix;
+    g.tiles = plasma_panel_tiles(A, up, k);
+    g.L = (const float *)plasma_tile_addr(A, k, k);
     g.W = (const float *)inv + k * mb * mb;
-    g.A0 = tile(k + 1);
-    g.A1 = tile(A.mt - 1);
-    // tiles k + 1 .. mt - 2 are whole: their addresses are a polynomial of
-    // degree 2 in m (linear but for the packed columns of upper storage)
-    g.step = g.ntiles > 2 ? tile(k + 2) - g.A0 : 0;
-    g.step2 = g.ntiles > 3 ? tile(k + 3) - 2 * (tile(k + 2) - g.A0) - g.A0
-                           : 0;
     g.P = (float *)panel + (size_t)(k - pbase) * mb * pcols +
           (size_t)pcol * mb;
     g.pstep = (ptrdiff_t)mb * pcols;
     g.ldl = plasma_tile_mmain(A, k);
-    g.lda = up ? g.ldl : plasma_tile_mmain(A, k + 1);
-    g.lda1 = up ? g.ldl : plasma_tile_mmain(A, A.mt - 1);
     g.ldp = A.mb;
     g.nb = A.mb;                        // tile k is not the last one
-    g.rows1 = plasma_tile_mview(A, A.mt - 1);
     g.status = status;
+    const plasma_panel_tiles_t &t = g.tiles;
     const bool full = A.mb == (small ? 64 : 128);
-    const bool vec = ((uintptr_t)g.L | (uintptr_t)g.A0 | (uintptr_t)g.A1) %
-                             16 == 0 && (g.ldl | g.lda | g.lda1) % 4 == 0 &&
-                     g.step % 4 == 0 && g.step2 % 4 == 0;
+    const bool vec = ((uintptr_t)g.A | (uintptr_t)g.L) % 16 == 0 &&
+                     (t.first | t.last) % 4 == 0 &&
+                     (t.step | t.step2) % 4 == 0 &&
+                     (g.ldl | t.ld | t.ld_last) % 4 == 0;
     const void *fn = up ? (small ? kernel_of<true, 4>(full, vec)
                                  : kernel_of<true, 8>(full, vec))
                         : (small ? kernel_of<false, 4>(full, vec)
                                  : kernel_of<false, 8>(full, vec));
-    const dim3 grid(g.ntiles, (A.mb + SP_ROWS - 1) / SP_ROWS);
+    const dim3 grid(t.ntiles, (A.mb + SP_ROWS - 1) / SP_ROWS);
     void *args[] = {&g};
     return hipLaunchKernel(fn, grid, dim3(SP_NT), args, 0, s) == hipSuccess
                ? 0 : PlasmaErrorInternal;
