@@ -27,8 +27,11 @@
 // 2.9 ms; per tile and sweep about 4.5 us in FP32 and 8.7 us in FP64.  Whole
 // solves, per-step form and this one: dposv n = 300 346, 277 us; n = 2000 and
 // nrhs 128 1721, 1266 us; n = 16384 and nrhs 128 42.0, 38.7 ms; sposv n =
-// 8192 6.73, 4.99 ms.  It wins at every order up to FLOW_SWEEP_NRHS = 128
-// right-hand sides; beyond, L is read too often (once per 16 of them).
+// 8192 6.73, 4.99 ms.  It is used up to FLOW_SWEEP_NRHS = 128 right-hand sides,
+// which is not where it stops winning, although it reads L once per 16 of them:
+// potrs n = 2000 with 256 and 768 right-hand sides 826, 368 and 954, 577 us; n =
+// 8192 3.89, 2.51 and 6.18, 6.00 ms; in FP32 n = 8192 2.97, 1.35 and 4.10, 3.03
+// ms.
 //
 // Eight waves; wave w holds rows 16 w .. of the block row (tiles of order
 // <= 128).  The operand that MFMA needs row by row (L or W) goes straight

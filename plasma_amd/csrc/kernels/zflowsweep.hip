@@ -17,8 +17,10 @@
 // (zchol.hip, two dependent launches of about 40 us per tile and sweep) 6.4
 // ms.  Whole solves, per-step form and this one: n = 300, nrhs 3 843, 596 us;
 // n = 2000, nrhs 128 5.60, 3.49 ms; n = 10000, nrhs 128 60.6, 49.7 ms; cposv
-// n = 4000, nrhs 32 8.99, 5.97 ms.  Up to ZFLOW_SWEEP_NRHS = 128 right-hand
-// sides, the largest measured; L is read once per 8 of them.
+// n = 4000, nrhs 32 8.99, 5.97 ms.  It is used up to ZFLOW_SWEEP_NRHS = 128
+// right-hand sides, which is not where it stops winning, although it reads L once
+// per 8 of them: potrs n = 2000 with 256 and 768 right-hand sides 2.89, 0.86 and
+// 3.04, 1.48 ms; n = 5000 7.46, 2.84 and 9.88, 6.85 ms.
 #include "common.hip.h"
 #include "directgemm.hip.h"
 #include "plasma_kernels.h"
